@@ -8,6 +8,8 @@ import torch
 
 import oracle
 from oracle import omnivoice as O
+from oracle import reference as R
+from tests.conftest import assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +43,55 @@ def test_conv_transpose1d_tiles_match_oracle(device, length, ci, co, k, stride, 
     mag = O.conv_transpose1d_ref(np.abs(x.cpu().numpy()).transpose(0, 2, 1), np.abs(dense), np.abs(bias), k, stride,
                                  pad, opad).transpose(0, 2, 1)
     assert (np.abs(y - ref) <= (n + 2) * 2.0 ** -24 * mag).all()
+
+
+# channels down to 8 (padded column tiles and channel steps), one frame, a frame count past a row tile,
+# channel slabs split over 1, 2 and 4 waves (wide first layers, few rows), more rows than one block takes
+@pytest.mark.parametrize("books,dim,latent,hidden,channels,strides,frames", [
+    (3, 32, 64, 64, 64, (3, 2, 2), 1), (1, 64, 192, 128, 256, (2, 3), 33), (2, 32, 128, 320, 512, (8, 5, 4, 2, 3), 3),
+    (4, 32, 64, 64, 96, (5, 7), 70)])
+def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, channels, strides, frames):
+    """Every stage of the fused decode against the float64 oracle over the stage's own input, and the waveform of
+    the run that keeps no stages against the run that does (the same arithmetic, so the same bits)."""
+    from torch2vk_amd.omnivoice.decoder import AudioDecoderConfig, OmniVoiceAudioDecoder, out_len, synthetic_dense
+
+    cfg = AudioDecoderConfig(codebooks=books, vocab=16, codebook_dim=dim, latent=latent, hidden=hidden,
+                             channels=channels, strides=strides)
+    dense = synthetic_dense(cfg, seed=frames)
+    dec = OmniVoiceAudioDecoder(cfg, dense, device)
+    assert dec._plan is not None
+    deq = {}
+    for n, a in dense.items():
+        if a.ndim != 2:
+            deq[n] = a.astype(np.float64)
+            continue
+        kp = (a.shape[1] + 31) // 32 * 32
+        deq[n] = oracle.dequant_q8_0(dec.w[n].cpu().numpy(), kp)[:, :a.shape[1]].astype(np.float64)
+        if not (n.startswith("cb") or n.endswith("convt.w")):
+            deq[n] = R.bf16_round(deq[n].astype(np.float32)).astype(np.float64)
+    bf = lambda a: R.bf16_round(np.asarray(a, np.float32)).astype(np.float64)  # noqa: E731
+    codes = np.random.default_rng(8).integers(-1, cfg.vocab + 1, (books, frames)).astype(np.int64)
+    stages = []
+    y = dec.decode(torch.from_numpy(codes), stages=stages)
+    assert torch.equal(y, dec.decode(torch.from_numpy(codes)))
+    y = y.cpu().numpy()
+    assert y.shape == (out_len(cfg, frames),)
+    got = [a.cpu().numpy().astype(np.float64)[0].T[None] for a in stages]
+    # ids outside the table embed as zeros: one zero row after the table
+    ref_deq = {n: (np.concatenate([a, np.zeros((1, a.shape[1]))]) if n.startswith("cb") else a) for n, a in deq.items()}
+    ids = np.where((codes >= 0) & (codes < cfg.vocab), codes, cfg.vocab)
+    checks = [("front", got[0], O.audio_decode_front_ref(cfg, ref_deq, ids, bf))]
+    k = 1
+    for i in range(len(strides)):
+        checks.append((f"block {i} upsample", got[k], O.audio_decode_upsample_ref(cfg, deq, got[k - 1], i)))
+        k += 1
+        for j, d in enumerate((1, 3, 9)):
+            checks.append((f"block {i} unit {j}", got[k],
+                           O.audio_decode_unit_ref(deq, got[k - 1], f"b{i}.r{j}.", d, bf)))
+            k += 1
+    checks.append(("final", y, O.audio_decode_final_ref(deq, got[-1], bf)))
+    # a stage holds up to two convolutions (the front three products): an fp32 sum that lands on the other side of
+    # a bf16 boundary moves one staged input by 2^-8 of itself, so the stage by 2^-8 of one product of its sums
+    for what, a, b in checks:
+        assert a.shape == b.shape, what
+        assert_close(a, b, max_abs=2.0 ** -8 * float(np.abs(b).max()), min_cos=0.99999, what=what)

@@ -16,7 +16,7 @@
 //
 // All of them are HBM-bound byte movers: coalesced 4- to 16-byte accesses,
 // one pass, no LDS.
-#include "common.h"
+#include "codec.h"
 
 namespace t2h {
 
@@ -436,8 +436,7 @@ __global__ __launch_bounds__(256) void snake_kernel(const float* __restrict__ x,
     if (i >= n) return;
     const float a = alpha[i % channels];
     const float v = x[i];
-    const float s = sinf(a * v);
-    y[i] = v + (1.0f / (a + eps)) * (s * s);
+    y[i] = snake_f32(v, a, eps);
 }
 
 extern "C" int t2h_snake(const float* x, const float* alpha, float* out, uint64_t rows, uint32_t channels, float eps,

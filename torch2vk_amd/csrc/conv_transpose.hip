@@ -10,7 +10,7 @@
 // As a product it is G[i, e] = sum_ci x[i, ci] W[ci, e], e = co K + k, followed by a fold that adds, for an
 // output position u = t + pad, the entries k = u % stride, k + stride, ... of rows i = u / stride, i - 1, ...
 // Everything stays fp32: weights d * q, inputs, products and sums (v_mfma_f32_32x32x2_f32).
-#include "common.h"
+#include "codec.h"
 
 namespace t2h {
 
@@ -29,6 +29,9 @@ struct ConvTArgs {
     uint32_t halo;          // rows of G before an output's own that its taps reach: ceil(K / stride) - 1
     int32_t i_first;        // pad / stride, the row of the first output
     uint32_t vec;           // x rows can be read 4 channels at a time
+    uint16_t* snaked;       // bf16 [B, L_out, Co] of snake(y, alpha), or null
+    const float* alpha;
+    float eps;
 };
 
 // One block: 32 rows i (the first `halo` of them only feed the others' outputs) x nt column tiles of 32
@@ -142,6 +145,7 @@ __global__ __launch_bounds__(CT_MAX_NT * 64) void conv_transpose1d_tile_kernel(c
     const uint32_t nco = 32 * nt / a.kh, cl = tid % nco, co = 32 * eb0 / a.kh + cl;
     if (co >= a.co) return;
     const float bias = a.bias ? a.bias[co] : 0.0f;
+    const float alpha = a.snaked ? a.alpha[co] : 0.0f;
     const uint32_t drow = 2 * a.kh / a.stride, dphase = 2 * a.kh % a.stride;
     uint32_t row = a.halo + tid / nco / a.stride, phase = tid / nco % a.stride;
     for (; row < CT_ROWS; row += drow, phase += dphase) {
@@ -157,7 +161,9 @@ __global__ __launch_bounds__(CT_MAX_NT * 64) void conv_transpose1d_tile_kernel(c
             const int i = i0 + (int)gr;  // rows outside the input are no taps (not zeros: 0 * inf)
             if (i >= 0 && i < (int)a.li) v += bs[gr * brow + cl * a.kh + k];
         }
-        a.out[((uint64_t)blockIdx.z * a.lo + (uint64_t)t) * a.co + co] = v;
+        const uint64_t at = ((uint64_t)blockIdx.z * a.lo + (uint64_t)t) * a.co + co;
+        a.out[at] = v;
+        if (a.snaked) a.snaked[at] = (uint16_t)f32_to_bf16_bits(snake_f32(v, alpha, a.eps));
     }
 }
 
@@ -190,6 +196,7 @@ __global__ __launch_bounds__(256) void conv_transpose1d_q8_0_kernel(const ConvTA
         }
     }
     a.out[idx] = acc;
+    if (a.snaked) a.snaked[idx] = (uint16_t)f32_to_bf16_bits(snake_f32(acc, a.alpha[co], a.eps));
 }
 
 static uint32_t ct_gcd(uint32_t a, uint32_t b) {
@@ -209,13 +216,10 @@ static uint32_t ct_tiles(uint32_t kh) {
     return base * (base >= 4 ? 1 : (4 + base - 1) / base);
 }
 
-}  // namespace t2h
-
-using namespace t2h;
-
-extern "C" int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_strides, const void* w, const float* bias,
-                                         float* out, uint32_t batch, uint32_t ci, uint32_t li, uint32_t co,
-                                         uint32_t kh, uint32_t stride, uint32_t pad, uint32_t lo, void* stream) {
+int conv_transpose1d_q8_0_launch(const float* x, const int64_t* x_strides, const void* w, const float* bias,
+                                 float* out, uint32_t batch, uint32_t ci, uint32_t li, uint32_t co, uint32_t kh,
+                                 uint32_t stride, uint32_t pad, uint32_t lo, uint16_t* snaked, const float* alpha,
+                                 float eps, void* stream) {
     if (!x || !x_strides || !w || !out) return T2H_ERR_NULL;
     if (ci == 0 || co == 0 || kh == 0 || stride == 0 || li == 0) return T2H_ERR_SHAPE;
     // L_out of a transposed conv plus an output padding in [0, stride): the extra last positions take the taps
@@ -241,6 +245,9 @@ extern "C" int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_stride
     a.stride = stride;
     a.pad = pad;
     a.lo = lo;
+    a.snaked = snaked;
+    a.alpha = alpha;
+    a.eps = eps;
     a.row_bytes = (uint32_t)(((uint64_t)co * kh + 31) / 32 * 34);
     a.n = (uint64_t)batch * lo * co;
     if (a.n == 0) return T2H_OK;
@@ -266,4 +273,13 @@ extern "C" int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_stride
     hipLaunchKernelGGL(conv_transpose1d_q8_0_kernel, dim3((uint32_t)((a.n + 255) / 256)), dim3(256), 0, s, a);
     T2H_LAUNCH_CHECK();
     return T2H_OK;
+}
+
+}  // namespace t2h
+
+extern "C" int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_strides, const void* w, const float* bias,
+                                         float* out, uint32_t batch, uint32_t ci, uint32_t li, uint32_t co,
+                                         uint32_t kh, uint32_t stride, uint32_t pad, uint32_t lo, void* stream) {
+    return t2h::conv_transpose1d_q8_0_launch(x, x_strides, w, bias, out, batch, ci, li, co, kh, stride, pad, lo,
+                                             nullptr, nullptr, 0.0f, stream);
 }

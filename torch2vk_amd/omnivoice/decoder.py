@@ -15,13 +15,15 @@ conv_transpose1d (each row padded to whole 32-value blocks).
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
 import numpy as np
 import torch
 
-from torch2vk_amd import kernels
+from torch2vk_amd import _lib, kernels
+from torch2vk_amd._lib import call, ptr, stream_handle
 
 DILATIONS = (1, 3, 9)
 
@@ -94,12 +96,80 @@ def quantize_rows(w: np.ndarray, device) -> torch.Tensor:
     return kernels.quantize(torch.from_numpy(full).to(device), "q8_0")
 
 
+def conv_fragments(rows: list[torch.Tensor], cin: int, taps: int) -> torch.Tensor:
+    """Q8_0 conv rows [n, cin * taps] (element c * taps + k), several matrices' inputs side by side, as the bf16
+    fragments t2h_codec_decode reads: [tap][step of 16 inputs][tile of 32 columns][64][8]."""
+    n, steps = int(rows[0].shape[0]), -(-cin // 32) * 2
+    out = torch.empty(taps, steps * len(rows), -(-n // 64) * 2, 64, 8, dtype=torch.bfloat16, device=rows[0].device)
+    for i, r in enumerate(rows):
+        call("t2h_conv_fragments_q8_0", ptr(r), n, cin, taps, steps * len(rows), steps * i, ptr(out), stream_handle())
+    return out
+
+
 class OmniVoiceAudioDecoder:
+    """``w`` holds the packed weights.  The convolutions are also laid out as bf16 fragments when the decoder is
+    made (t2h_codec_decode then runs a whole decode as about 40 launches); channel counts that path is not built
+    for run operator by operator."""
+
     def __init__(self, cfg: AudioDecoderConfig, dense: dict[str, np.ndarray], device) -> None:
         self.cfg = cfg
         self.device = torch.device(device)
         self.w = {n: (quantize_rows(a, self.device) if a.ndim == 2 else torch.from_numpy(a).to(self.device))
                   for n, a in dense.items()}
+        self._dims = (ctypes.c_uint32 * (7 + len(cfg.strides)))(cfg.codebooks, cfg.vocab, cfg.codebook_dim, cfg.latent,
+                                                                cfg.hidden, cfg.channels, len(cfg.strides), *cfg.strides)
+        fused = cfg.codebook_dim % 32 == 0 and cfg.latent % 64 == 0 and cfg.hidden % 64 == 0 and \
+            self._workspace_bytes(1) > 0
+        self._plan = self._lay_out() if fused else None
+
+    def _lay_out(self) -> list[torch.Tensor]:
+        """t2h_codec_decode's operands in its order."""
+        cfg, w = self.cfg, self.w
+        bias = w["proj0.b"]
+        for c in range(1, cfg.codebooks):
+            bias = bias + w[f"proj{c}.b"]
+        plan = [w[f"cb{c}"] for c in range(cfg.codebooks)]
+        plan += [conv_fragments([w[f"proj{c}.w"] for c in range(cfg.codebooks)], cfg.codebook_dim, 1), bias]
+        plan += [conv_fragments([w["fc2.w"]], cfg.latent, 1), w["fc2.b"]]
+        plan += [conv_fragments([w["conv1.w"]], cfg.hidden, 7), w["conv1.b"], w["b0.alpha"]]
+        ch, blocks, units = cfg.channels, len(cfg.strides), len(DILATIONS)
+        for i in range(blocks):
+            ch //= 2
+            plan += [w[f"b{i}.convt.w"], w[f"b{i}.convt.b"], w[f"b{i}.r0.a1"]]
+            for j in range(units):
+                p = f"b{i}.r{j}."
+                if j + 1 < units:
+                    after = f"b{i}.r{j + 1}.a1"
+                else:
+                    after = f"b{i + 1}.alpha" if i + 1 < blocks else "final.alpha"
+                plan += [conv_fragments([w[p + "c1.w"]], ch, 7), w[p + "c1.b"], w[p + "a2"],
+                         conv_fragments([w[p + "c2.w"]], ch, 1), w[p + "c2.b"], w[after]]
+        return plan + [conv_fragments([w["conv2.w"]], ch, 7), w["conv2.b"]]
+
+    def _workspace_bytes(self, frames: int) -> int:
+        """Bytes t2h_codec_decode needs (0: more frames than it takes)."""
+        return int(_lib.lib().t2h_codec_decode_workspace_bytes(ctypes.addressof(self._dims), frames))
+
+    def _decode_fused(self, codes: torch.Tensor, nbytes: int, stages: list | None) -> torch.Tensor:
+        cfg, t = self.cfg, int(codes.shape[1])
+        codes = codes[:cfg.codebooks].contiguous()
+        space = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        out = torch.empty(out_len(cfg, t), dtype=torch.float32, device=self.device)
+        operands = (ctypes.c_void_p * len(self._plan))(*[x.data_ptr() for x in self._plan])
+        stage_ptrs = None
+        if stages is not None:
+            ch, length = cfg.channels, t
+            new = [torch.empty(1, t, ch, dtype=torch.float32, device=self.device)]
+            for s in cfg.strides:
+                ch, length = ch // 2, length * s
+                new += [torch.empty(1, length, ch, dtype=torch.float32, device=self.device)
+                        for _ in range(1 + len(DILATIONS))]
+            stages.extend(new)
+            stage_arr = (ctypes.c_void_p * len(new))(*[x.data_ptr() for x in new])
+            stage_ptrs = ctypes.addressof(stage_arr)
+        call("t2h_codec_decode", ctypes.addressof(self._dims), ctypes.addressof(operands), len(self._plan), ptr(codes), t, kernels.SNAKE_EPS,
+             ptr(out), stage_ptrs, ptr(space), nbytes, stream_handle())
+        return out
 
     def _unit(self, x: torch.Tensor, p: str, dil: int) -> torch.Tensor:
         w = self.w
@@ -115,6 +185,10 @@ class OmniVoiceAudioDecoder:
         cfg, w = self.cfg, self.w
         codes = codes.to(device=self.device, dtype=torch.int64)
         t = int(codes.shape[1])
+        if self._plan is not None and 0 < t < 1 << 31 and codes.dim() == 2 and codes.shape[0] >= cfg.codebooks:
+            nbytes = self._workspace_bytes(t)
+            if nbytes:
+                return self._decode_fused(codes, nbytes, stages)
         acc = torch.zeros(t, cfg.latent, dtype=torch.float32, device=self.device)
         for c in range(cfg.codebooks):
             e = kernels.embedding_q8_0(w[f"cb{c}"], codes[c].contiguous(), cfg.codebook_dim)
