@@ -163,6 +163,13 @@ int t2h_q4k_gemm(const void* x, const void* w, void* y, int out_dtype, const flo
  * text_layer.py; src/models/optimized_qwen3/shaders/swiglu_f32.py). */
 int t2h_gemm_swiglu(int wtype, const void* x, const void* w_gate, const void* w_up, void* y, uint32_t m, uint32_t k,
                     uint32_t n_ff, void* stream);
+/* The same products for few rows, in one launch of small tiles (any m, n; k % 64 == 0): y[m, n] = act(x . deq(W)^T +
+ * bias) (+ residual), or with w_up the SwiGLU form of t2h_gemm_swiglu (n features, bf16 out).  tile: 0: 32 x 32
+ * outputs a block, 1: 64 x 32, 2: 64 x 64, 3: 128 x 64 (2 and 3 only for the SwiGLU form).  Operands, rounding and
+ * status codes as t2h_q8_0_linear / t2h_gemm_swiglu; sums differ from theirs by fp32 order. */
+int t2h_gemm_tiles(int wtype, const void* x, const void* w, const void* w_up, const float* bias, int act, void* y,
+                   int out_dtype, const float* residual, uint32_t m, uint32_t k, uint32_t n, uint32_t w_k,
+                   uint32_t tile, void* stream);
 /* Split-K form of the prefill GEMMs above, for grids too small to fill the GPU (a few hundred rows, as in a
  * short prompt or a 512-token prefill chunk): K is cut into `splits` equal parts of whole 64-wide stages, each
  * part's fp32 products go to partials (t2h_gemm_splitk_bytes(m, n, splits, swiglu) bytes, 16-B aligned),
