@@ -191,7 +191,7 @@ __global__ __launch_bounds__(WPB * 64) void q4k_gemv_kernel(const Q4GemvArgs a) 
                          bf16_round(hv[j].z * inv * wv[j].z), bf16_round(hv[j].w * inv * wv[j].w));
         }
     } else {
-        const uint16_t* xb = reinterpret_cast<const uint16_t*>(a.x);
+        const uint16_t* xb = reinterpret_cast<const uint16_t*>(a.x) + (size_t)blockIdx.y * K;
         uint2 xv[PT];
 #pragma unroll
         for (int j = 0; j < PT; ++j) {
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(WPB * 64) void q4k_gemv_kernel(const Q4GemvArgs a) 
         pi += (a.n_parts > 1 && row >= a.parts[1].row_begin) ? 1 : 0;
         pi += (a.n_parts > 2 && row >= a.parts[2].row_begin) ? 1 : 0;
         const Q4Part& p = a.parts[pi];
-        const uint32_t local = row - p.row_begin;
+        const size_t local = (size_t)blockIdx.y * p.n + (row - p.row_begin);  // token blockIdx.y (one part then)
         if constexpr (EPI == Q4EPI_F32) {
             reinterpret_cast<float*>(p.y)[local] = v;
         } else if constexpr (EPI == Q4EPI_BF16) {
@@ -487,7 +487,7 @@ extern "C" int t2h_set_gemv_max_blocks(uint32_t max_blocks, uint32_t max_blocks_
 
 // Launch over `max_blocks` (or exactly `fixed_blocks` blocks when non-zero).
 static int q4k_launch(int pro, int epi, Q4GemvArgs a, uint32_t nsb, uint32_t max_blocks, uint32_t fixed_blocks,
-                      hipStream_t s) {
+                      hipStream_t s, uint32_t tokens = 1) {
     if (a.n_units == 0) return T2H_OK;
     const Q4Geometry geo = q4_geometry(nsb, epi);
     uint32_t blocks;
@@ -499,7 +499,7 @@ static int q4k_launch(int pro, int epi, Q4GemvArgs a, uint32_t nsb, uint32_t max
         a.units_per_wave = units_per_wave_for(a.n_units, max_blocks ? max_blocks : 1u, geo);
         blocks = blocks_for(a.n_units, a.units_per_wave, geo);
     }
-    const dim3 grid(blocks);
+    const dim3 grid(blocks, tokens);
     const uint32_t upw = q4_straight_line(nsb, epi) && a.units_per_wave <= 4 ? a.units_per_wave : 0;
     hipError_t e = hipErrorInvalidValue;
     if (pro == Q4PRO_BF16) {
@@ -574,7 +574,11 @@ extern "C" int t2h_q4k_matvec(const void* x, const void* w, void* y, int out_dty
     if (n % rpw != 0) return T2H_ERR_SHAPE;
     const size_t out_size = out_dtype == T2H_DTYPE_F32 ? 4 : 2;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    for (uint32_t row = 0; row < m; ++row) {
+    // Every token in one launch, blockIdx.y its row: the tokens' blocks run side by side, so the weights come from
+    // HBM once and from L2 for the others (block x of every token runs on the same XCD where the grid is a multiple
+    // of 8 blocks), and one token's latencies hide the next's.  6 tokens of K 4096, N 4096: 9.9 us (20.3 as 6
+    // launches), of K 1024, N 3072: 4.5 (16.1).
+    for (uint32_t row = 0; row < m; row += 65535) {
         Q4GemvArgs a = {};
         const void* wv[1] = {w};
         void* yv[1] = {reinterpret_cast<uint8_t*>(y) + (size_t)row * n * out_size};
@@ -584,7 +588,7 @@ extern "C" int t2h_q4k_matvec(const void* x, const void* w, void* y, int out_dty
         a.x = reinterpret_cast<const uint16_t*>(x) + (size_t)row * k;
         a.residual = residual ? residual + (size_t)row * n : nullptr;
         a.n_units = total / rpw;
-        st = q4k_launch(Q4PRO_BF16, epi, a, nsb, g_max_blocks, 0, s);
+        st = q4k_launch(Q4PRO_BF16, epi, a, nsb, g_max_blocks, 0, s, m - row < 65535u ? m - row : 65535u);
         if (st) return st;
     }
     return T2H_OK;

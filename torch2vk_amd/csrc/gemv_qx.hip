@@ -221,7 +221,7 @@ __global__ __launch_bounds__(QX_THREADS) void qx_gemv_kernel(const QxArgs a) {
             v[0] = h0.x * inv * w0.x; v[1] = h0.y * inv * w0.y; v[2] = h0.z * inv * w0.z; v[3] = h0.w * inv * w0.w;
             v[4] = h1.x * inv * w1.x; v[5] = h1.y * inv * w1.y; v[6] = h1.z * inv * w1.z; v[7] = h1.w * inv * w1.w;
         } else {
-            const uint4 r = load_u4(reinterpret_cast<const uint16_t*>(a.x) + c * 8);
+            const uint4 r = load_u4(reinterpret_cast<const uint16_t*>(a.x) + (size_t)blockIdx.y * K + c * 8);
             const uint32_t u[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(QX_THREADS) void qx_gemv_kernel(const QxArgs a) {
             float v = res[0];
 #pragma unroll
             for (int r = 1; r < RPW; ++r) v = (lane == r) ? res[r] : v;
-            const uint32_t row = row0 + lane;
+            const size_t row = (size_t)blockIdx.y * (a.n_units * RPW) + (row0 + lane);  // token blockIdx.y
             if constexpr (EPI == QXEPI_F32) {
                 reinterpret_cast<float*>(a.y)[row] = v;
             } else if constexpr (EPI == QXEPI_BF16) {
@@ -416,7 +416,8 @@ static uint32_t qx_pick_blocks(uint32_t n_units, uint32_t max_blocks) {
 constexpr uint32_t QX_MAX_BLOCKS = 256;
 
 template <class F>
-static int qx_run(int pro, int epi, QxArgs a, const QxGeom& g, uint32_t n, uint32_t blocks, hipStream_t s) {
+static int qx_run(int pro, int epi, QxArgs a, const QxGeom& g, uint32_t n, uint32_t blocks, hipStream_t s,
+                  uint32_t tokens = 1) {
     if (n % g.rpw != 0) return T2H_ERR_SHAPE;
     a.pieces = g.pieces;
     a.row_bytes = a.k / F::BLOCK_VALUES * F::BLOCK_BYTES;
@@ -424,7 +425,7 @@ static int qx_run(int pro, int epi, QxArgs a, const QxGeom& g, uint32_t n, uint3
     if (a.n_units == 0) return T2H_OK;
     if (blocks == 0) blocks = qx_pick_blocks(a.n_units, QX_MAX_BLOCKS);
     a.units_per_wave = qx_units_per_wave(a.n_units, blocks);
-    const dim3 grid(blocks);
+    const dim3 grid(blocks, tokens);
     hipError_t e = hipErrorInvalidValue;
     if (pro == QXPRO_BF16) {
         switch (epi) {
@@ -445,7 +446,8 @@ static int qx_run(int pro, int epi, QxArgs a, const QxGeom& g, uint32_t n, uint3
     return e == hipSuccess ? T2H_OK : T2H_ERR_HIP_BASE + (int)e;
 }
 
-// y = [RMSNorm](x) . deq(W)^T [+ residual], one launch per token row
+// y = [RMSNorm](x) . deq(W)^T [+ residual]; every token in one launch, blockIdx.y its row (as t2h_q4k_matvec; the
+// RMSNorm prologue takes one)
 template <class F>
 static int qx_matvec(const void* x, const float* norm_w, float eps, const void* w, void* y, int out_dtype,
                      const float* residual, uint32_t m, uint32_t k, uint32_t n, void* stream) {
@@ -468,7 +470,7 @@ static int qx_matvec(const void* x, const float* norm_w, float eps, const void* 
     }
     const size_t x_size = norm_w ? 4 : 2;
     const size_t out_size = out_dtype == T2H_DTYPE_F32 ? 4 : 2;
-    for (uint32_t row = 0; row < m; ++row) {
+    for (uint32_t row = 0; row < m; row += 65535) {
         QxArgs a = {};
         a.x = reinterpret_cast<const uint8_t*>(x) + (size_t)row * k * x_size;
         a.norm_w = norm_w;
@@ -477,7 +479,8 @@ static int qx_matvec(const void* x, const float* norm_w, float eps, const void* 
         a.w = reinterpret_cast<const uint8_t*>(w);
         a.y = reinterpret_cast<uint8_t*>(y) + (size_t)row * n * out_size;
         a.k = k;
-        st = qx_run<F>(norm_w ? QXPRO_RMSNORM : QXPRO_BF16, epi, a, g, n, 0, reinterpret_cast<hipStream_t>(stream));
+        st = qx_run<F>(norm_w ? QXPRO_RMSNORM : QXPRO_BF16, epi, a, g, n, 0, reinterpret_cast<hipStream_t>(stream),
+                       m - row < 65535u ? m - row : 65535u);
         if (st) return st;
     }
     return T2H_OK;

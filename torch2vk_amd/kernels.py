@@ -480,7 +480,7 @@ def quantized_linear(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch
                      out_dtype: torch.dtype = torch.float32, residual: torch.Tensor | None = None) -> torch.Tensor:
     """y[M, N] = x[M, K] . deq(W)^T (+ residual) with the kernel the reference would pick: the weight's GGUF type
     selects the family (run_quantized_linear, src/torch2vk/runtime/quantized_dispatch.py:15-35) and M <= 8 rows
-    run the decode GEMV (one launch per row, the weights streamed per row), more the matrix-core GEMM
+    run the decode GEMV (all rows in one launch), more the matrix-core GEMM
     (make_linear_nobias_q4_k_m_variant, src/torch2vk/export/shaders/linear_nobias_quantized.py:47-80).
     Shapes the GEMVs are not built for (matvec_supported) run on the GEMM at any M."""
     if wtype not in ("q4_k", "q6_k", "q8_0"):
