@@ -21,6 +21,7 @@ Q6_K_BYTES = 210
 Q8_0_BYTES = 34
 RMS_EPS = 1e-6
 
+_OUT_DTYPE_TUPLE = (torch.float32, torch.bfloat16)
 _OUT_DTYPES = {torch.float32: T2H_DTYPE_F32, torch.bfloat16: T2H_DTYPE_BF16}
 # the reference's uint32 buffers (token ids of the LM head's partials, done / length / stopped flags), or
 # int32 ones of the same bits
@@ -30,6 +31,9 @@ WTYPES = {"q4_k": _lib.T2H_WTYPE_Q4_K, "q6_k": _lib.T2H_WTYPE_Q6_K, "q8_0": _lib
 
 
 def _check(t: torch.Tensor, name: str, dtype: torch.dtype | tuple[torch.dtype, ...], *, align: int = 16) -> None:
+    if (isinstance(t, torch.Tensor) and t.is_cuda and (t.dtype is dtype or type(dtype) is tuple and t.dtype in dtype)
+            and t.is_contiguous() and t.data_ptr() % align == 0):
+        return  # what follows only names the fault (about 0.7 us less a launch of three or four tensors)
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
     if t.device.type != "cuda":
@@ -108,7 +112,7 @@ def q4k_matvec(x: torch.Tensor, w: torch.Tensor, *, out: torch.Tensor | None = N
     n = _check_q4(w, "weight", None, k)
     if out is None:
         out = torch.empty(*x.shape[:-1], n, dtype=out_dtype, device=x.device)
-    _check(out, "output", tuple(_OUT_DTYPES), align=4)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=4)
     if out.numel() != m * n:
         raise ValueError(f"output has {out.numel()} elements, expected {m * n}")
     if residual is not None:
@@ -264,7 +268,7 @@ def qx_matvec(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor
     n = _check_packed(w, "weight", wtype, k)
     if out is None:
         out = torch.empty(*x.shape[:-1], n, dtype=out_dtype, device=x.device)
-    _check(out, "output", tuple(_OUT_DTYPES), align=4)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=4)
     if out.numel() != m * n:
         raise ValueError(f"output has {out.numel()} elements, expected {m * n}")
     if residual is not None:
@@ -393,7 +397,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor | No
     n = _check_packed(w, "weight", wtype, k)
     if out is None:
         out = torch.empty(*x.shape[:-1], n, dtype=out_dtype, device=x.device)
-    _check(out, "output", tuple(_OUT_DTYPES), align=4)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=4)
     if out.numel() != m * n:
         raise ValueError(f"output has {out.numel()} elements, expected {m * n}")
     if residual is not None:
@@ -584,7 +588,7 @@ def q8_0_linear(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None =
             raise ValueError(f"bias must have {n} elements, got {bias.numel()}")
     if out is None:
         out = torch.empty(*x.shape[:-1], n, dtype=out_dtype, device=x.device)
-    _check(out, "output", tuple(_OUT_DTYPES), align=4)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=4)
     if out.numel() != m * n:
         raise ValueError(f"output has {out.numel()} elements, expected {m * n}")
     if residual is not None:
@@ -886,6 +890,8 @@ def decode_layers_trace(layers: int, device) -> torch.Tensor:
 
 def _check_strided(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
     """Device, dtype and a contiguous last dimension; other strides are free (the kernel takes them)."""
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype and t.stride(-1) == 1:
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
     if t.device.type != "cuda":
@@ -896,6 +902,7 @@ def _check_strided(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
         raise ValueError(f"{name} needs a contiguous last dimension")
 
 
+_Strides12, _Strides14 = ctypes.c_int64 * 12, ctypes.c_int64 * 14
 FA_BLOCK_QUERIES = 128  # queries per flash-attention block (a row of mask tiles)
 FA_TILE_KEYS = 64       # keys per flash-attention tile
 
@@ -947,9 +954,7 @@ def flash_attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: t
             raise ValueError(f"mask must be [B or 1, {t_len}, {s_len}], got {tuple(mask.shape)}")
         m_sb = mask.stride(0) if mask.shape[0] == b else 0
         m_st = mask.stride(1)
-    strides = (_lib.ctypes.c_int64 * 14)(q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
-                                         k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0),
-                                         out.stride(1), out.stride(2), m_sb, m_st)
+    strides = _Strides14(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3], m_sb, m_st)
     if mask is not None and mask_tiles is not False:
         tiles = fa_mask_tiles(mask) if mask_tiles is None or mask_tiles is True else mask_tiles
         want = (mask.shape[0], -(-t_len // FA_BLOCK_QUERIES), -(-s_len // FA_TILE_KEYS))
@@ -995,9 +1000,7 @@ def flash_attn_segments(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_se
     _check_strided(out, "output", torch.bfloat16)
     if tuple(out.shape) != (b, t_len, nh, d):
         raise ValueError(f"output must be {(b, t_len, nh, d)}, got {tuple(out.shape)}")
-    strides = (_lib.ctypes.c_int64 * 12)(q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
-                                         k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0),
-                                         out.stride(1), out.stride(2))
+    strides = _Strides12(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3])
     call("t2h_flash_attn_segments", ptr(q), ptr(k), ptr(v), ptr(out), ptr(cu), cu.numel() - 1, b, nh, nk, t_len, d,
          strides, float(scale or 0.0), stream_handle())
     return out
@@ -1039,21 +1042,21 @@ def embedding_q4_k_seqs(w: torch.Tensor, ids: list[torch.Tensor], dim: int, outs
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None = None,
              eps: float = RMS_EPS) -> torch.Tensor:
-    _check(x, "x", tuple(_OUT_DTYPES), align=2)
+    _check(x, "x", _OUT_DTYPE_TUPLE, align=2)
     _check(weight, "weight", torch.float32, align=4)
     h = int(x.shape[-1])
     if weight.numel() != h:
         raise ValueError("weight must have H elements")
     if out is None:
         out = torch.empty_like(x)
-    _check(out, "output", tuple(_OUT_DTYPES), align=2)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=2)
     call("t2h_rms_norm", ptr(x), _OUT_DTYPES[x.dtype], ptr(weight), ptr(out), _OUT_DTYPES[out.dtype],
          x.numel() // h, h, eps, stream_handle())
     return out
 
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    _check(gate, "gate", tuple(_OUT_DTYPES), align=2)
+    _check(gate, "gate", _OUT_DTYPE_TUPLE, align=2)
     _check(up, "up", gate.dtype, align=2)
     if up.shape != gate.shape:
         raise ValueError("gate and up must have the same shape")
@@ -1112,7 +1115,7 @@ def im2col(x: torch.Tensor, kernel: tuple[int, int], stride: tuple[int, int] = (
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out: torch.Tensor | None = None, *,
                out_dtype: torch.dtype = torch.bfloat16, eps: float = 1e-5) -> torch.Tensor:
     """LayerNorm over the last dimension (LAYER_NORM_F32W_F32B_F32); x fp32 or bf16, out fp32 or bf16."""
-    _check(x, "x", tuple(_IN_DTYPES))
+    _check(x, "x", _OUT_DTYPE_TUPLE)
     cols = int(x.shape[-1])
     for t, name in ((weight, "weight"), (bias, "bias")):
         _check(t, name, torch.float32)
@@ -1120,7 +1123,7 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out: t
             raise ValueError(f"{name} must have {cols} elements")
     if out is None:
         out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _check(out, "output", tuple(_IN_DTYPES))
+    _check(out, "output", _OUT_DTYPE_TUPLE)
     if out.numel() != x.numel():
         raise ValueError("output must have x's shape")
     call("t2h_layer_norm", ptr(x), _IN_DTYPES[x.dtype], ptr(weight), ptr(bias), ptr(out), _IN_DTYPES[out.dtype],
@@ -1130,10 +1133,10 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out: t
 
 def gelu(x: torch.Tensor, out: torch.Tensor | None = None, *, out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """x * (1 + erf(x / sqrt 2)) / 2 (GELU_F32); x, out fp32 or bf16, numel % 4 == 0."""
-    _check(x, "x", tuple(_IN_DTYPES), align=8)
+    _check(x, "x", _OUT_DTYPE_TUPLE, align=8)
     if out is None:
         out = torch.empty(x.shape, dtype=out_dtype or x.dtype, device=x.device)
-    _check(out, "output", tuple(_IN_DTYPES), align=8)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=8)
     if out.numel() != x.numel():
         raise ValueError("output must have x's shape")
     if x.numel() % 4:
@@ -1364,9 +1367,9 @@ def rms_norm_rope(x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor, sin:
     """Per-head RMSNorm (D = 128) + RoPE from a table: x [B, T, G, D] fp32 / bf16, cos / sin fp32 [B, T, D] ->
     out [B, T, G, D], or [B, G, T, D] when ``transpose_out`` (RMS_NORM_ROPE_TRANSPOSE_F16,
     RMS_NORM_ROPE_TOKEN_F32)."""
-    _check(x, "x", tuple(_OUT_DTYPES), align=4)
+    _check(x, "x", _OUT_DTYPE_TUPLE, align=4)
     _check(weight, "weight", torch.float32, align=4)
-    _check(out, "output", tuple(_OUT_DTYPES), align=4)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=4)
     if x.dim() != 4:
         raise ValueError(f"x must be [B, T, G, D], got {tuple(x.shape)}")
     b, t_len, g, d = (int(v) for v in x.shape)
@@ -1387,7 +1390,7 @@ def rms_norm_rope(x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor, sin:
 def kv_cache_write(src: torch.Tensor, positions: torch.Tensor, caches: list[torch.Tensor]) -> None:
     """src [B, T, H, D] (fp32 or bf16) into each bf16 cache [B, S_c, H, D] at positions int64 [T]
     (TOKEN_MAJOR_KV_CACHE_WRITE_F16_PAIR / _TRIPLE, TOKEN_MAJOR_VALUE_CACHE_WRITE_F32_TO_F16_PAIR / _TRIPLE)."""
-    _check(src, "src", tuple(_OUT_DTYPES), align=4 if src.dtype == torch.bfloat16 else 8)
+    _check(src, "src", _OUT_DTYPE_TUPLE, align=4 if src.dtype == torch.bfloat16 else 8)
     _check(positions, "cache_position", torch.int64, align=8)
     if src.dim() != 4:
         raise ValueError(f"src must be [B, T, H, D], got {tuple(src.shape)}")
@@ -1425,7 +1428,7 @@ def token_select_chunks(scores: torch.Tensor, tokens: torch.Tensor, chunk_scores
 
 def add(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """out = x + y elementwise, fp32 or bf16 (ADD_F32_PREFILL, ADD_F32_36); out may be x or y."""
-    _check(x, "x", tuple(_OUT_DTYPES), align=2)
+    _check(x, "x", _OUT_DTYPE_TUPLE, align=2)
     _check(y, "y", x.dtype, align=2)
     if y.shape != x.shape:
         raise ValueError("x and y must have the same shape")
@@ -1441,7 +1444,7 @@ def add(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor | None = None) -> to
 def slice_last_token(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out [B, 1, H] = x[:, -1] of fp32 x [B, S, H] (SLICE_LAST_TOKEN_F32_TO_F16)."""
     _check(x, "x", torch.float32, align=4)
-    _check(out, "output", tuple(_OUT_DTYPES), align=2)
+    _check(out, "output", _OUT_DTYPE_TUPLE, align=2)
     if x.dim() != 3:
         raise ValueError(f"x must be [B, S, H], got {tuple(x.shape)}")
     b, s_len, h = (int(v) for v in x.shape)
