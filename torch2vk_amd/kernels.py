@@ -1112,6 +1112,71 @@ def im2col(x: torch.Tensor, kernel: tuple[int, int], stride: tuple[int, int] = (
     return out
 
 
+def conv2d_rows(w: torch.Tensor, channels: int, kernel: tuple[int, int]) -> torch.Tensor:
+    """Q8_0 conv2d rows (uint8 [N, 34 * blocks], element (c, ky, kx)) as ``conv2d``'s weights: bf16 [N, kp], element
+    (ky, kx, c), kp = kh * kw * channels rounded up to 64, zeros past them; each weight d * q rounded once to bf16, as
+    the GEMM's own operands are."""
+    n, taps = int(w.shape[0]), kernel[0] * kernel[1]
+    if w.dtype != torch.uint8 or tuple(w.shape) != (n, -(-channels * taps // 32) * Q8_0_BYTES):
+        raise ValueError(f"weight must be uint8 [N, 34 * ceil({channels * taps} / 32)], got {tuple(w.shape)}")
+    blocks = w.reshape(n, -1, Q8_0_BYTES)
+    d = blocks[..., :2].contiguous().view(torch.float16).float()
+    rows = (d * blocks[..., 2:].contiguous().view(torch.int8).float()).view(n, -1)[:, :channels * taps]
+    rows = rows.view(n, channels, taps).transpose(1, 2).reshape(n, -1).to(torch.bfloat16)
+    return torch.nn.functional.pad(rows, (0, -(channels * taps) % 64)).contiguous()
+
+
+def conv2d(x: torch.Tensor, w_rows: torch.Tensor, bias: torch.Tensor | None, kernel: tuple[int, int], stride: int,
+           pad: int, *, act: str | None = None, tile: int = -1) -> torch.Tensor:
+    """Channels-last conv2d as an implicit GEMM: x bf16 [B, H, W, C], ``w_rows`` from ``conv2d_rows``, bias fp32 [N] ->
+    bf16 [B, Ho, Wo, N].  C % 8 == 0, C >= 64, at most 24 taps."""
+    _check(x, "x", torch.bfloat16)
+    _check(w_rows, "weight rows", torch.bfloat16)
+    if x.dim() != 4:
+        raise ValueError(f"x must be [B, H, W, C], got {tuple(x.shape)}")
+    b, h, w, c = (int(v) for v in x.shape)
+    n = int(w_rows.shape[0])
+    kp = -(-kernel[0] * kernel[1] * c // 64) * 64
+    if tuple(w_rows.shape) != (n, kp):
+        raise ValueError(f"weight rows must be [N, {kp}], got {tuple(w_rows.shape)}")
+    if bias is not None:
+        _check(bias, "bias", torch.float32, align=4)
+        if bias.numel() != n:
+            raise ValueError(f"bias must have {n} elements, got {bias.numel()}")
+    if act not in ACTS:
+        raise ValueError(f"act must be one of {sorted(a for a in ACTS if a)} or None, got {act!r}")
+    out = torch.empty(b, conv_out_size(h, kernel[0], stride, pad), conv_out_size(w, kernel[1], stride, pad), n,
+                      dtype=torch.bfloat16, device=x.device)
+    call("t2h_conv2d_bf16", ptr(x), ptr(w_rows), ptr(bias), ACTS[act], ptr(out), b, h, w, c, n, *kernel, stride, pad,
+         tile, stream_handle())
+    return out
+
+
+def conv2d_1ch(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, kernel: tuple[int, int], stride: int,
+               pad: int, *, act: str | None = None) -> torch.Tensor:
+    """conv2d of one fp32 channel (rounded to bf16): x [B, 1, H, W], w Q8_0 rows [N, 34] of at most 16 taps, bias fp32
+    [N] -> channels-last bf16 [B, Ho, Wo, N].  N % 8 == 0."""
+    _check(x, "x", torch.float32, align=4)
+    _check(w, "weight", torch.uint8, align=2)
+    if x.dim() != 4 or x.shape[1] != 1:
+        raise ValueError(f"x must be [B, 1, H, W], got {tuple(x.shape)}")
+    b, _, h, width = (int(v) for v in x.shape)
+    n = int(w.shape[0])
+    if tuple(w.shape) != (n, Q8_0_BYTES):
+        raise ValueError(f"weight must be uint8 [N, {Q8_0_BYTES}], got {tuple(w.shape)}")
+    if bias is not None:
+        _check(bias, "bias", torch.float32, align=4)
+        if bias.numel() != n:
+            raise ValueError(f"bias must have {n} elements, got {bias.numel()}")
+    if act not in ACTS:
+        raise ValueError(f"act must be one of {sorted(a for a in ACTS if a)} or None, got {act!r}")
+    out = torch.empty(b, conv_out_size(h, kernel[0], stride, pad), conv_out_size(width, kernel[1], stride, pad), n,
+                      dtype=torch.bfloat16, device=x.device)
+    call("t2h_conv2d_1ch_q8_0", ptr(x), ptr(w), ptr(bias), ACTS[act], ptr(out), b, h, width, n, *kernel, stride, pad,
+         stream_handle())
+    return out
+
+
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out: torch.Tensor | None = None, *,
                out_dtype: torch.dtype = torch.bfloat16, eps: float = 1e-5) -> torch.Tensor:
     """LayerNorm over the last dimension (LAYER_NORM_F32W_F32B_F32); x fp32 or bf16, out fp32 or bf16."""
