@@ -1,0 +1,96 @@
+"""The prefill GEMM below 4096 rows by gemm_plan (K parts, weights dequantised first or in the loop) against the
+one-pass kernel over packed rows: the same bf16 operands, another fp32 order where K is split."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+
+@pytest.mark.parametrize("wtype", ["q4_k", "q6_k", "q8_0", "bf16"])
+@pytest.mark.parametrize("gated", [False, True])
+def test_plan_stays_in_the_kernels_limits(wtype, gated):
+    """Every part has at least two stages of K, splits stay in two rounds of blocks, and only packed rows are
+    dequantised."""
+    from torch2vk_amd import kernels
+
+    for m in (0, 1, 9, 128, 129, 520, 1024, 1901, 4095):
+        for n in (1, 7, 896, 4096, 12288, 151936):
+            for k in (64, 256, 896, 4096, 12288):
+                splits, dequant = kernels.gemm_plan(m, n, k, wtype, gated)
+                tiles = -(-m // 128) * -(-n * (2 if gated else 1) // 256)
+                assert splits == 1 or (splits <= min(16, k // 128) and tiles * splits <= 512)
+                assert not (dequant and wtype == "bf16")
+                assert kernels.gemm_plan(m, n, k, wtype, gated, False)[1] is False
+
+
+# each route past gemm_tile's tiles: in the loop and dequantised, one pass and split, ragged rows and columns
+@pytest.mark.gpu
+@pytest.mark.parametrize("wtype,m,n,k,gated,want", [
+    ("q4_k", 33, 4096, 6144, False, (16, False)), ("q4_k", 1037, 4099, 4096, False, None),
+    ("q4_k", 1900, 6000, 2048, True, (1, True)), ("q6_k", 735, 4096, 4096, False, (2, True)),
+    ("q6_k", 2049, 2050, 6144, False, (3, True)), ("q6_k", 300, 1030, 8192, True, None),
+    ("q8_0", 548, 4096, 4096, False, (3, False)), ("q8_0", 3000, 4100, 2048, False, (1, True)),
+    ("bf16", 548, 4096, 4096, False, (3, False))])
+def test_planned_gemm_equals_one_pass(device, wtype, m, n, k, gated, want):
+    from torch2vk_amd import kernels
+
+    plan = kernels.gemm_plan(m, n, k, wtype, gated)
+    print(f"{wtype} M={m} N={n} K={k} gated={gated} plan={plan}", flush=True)
+    assert kernels.gemm_tile(m, 2 * n if gated else n, k, gated) is None and plan == (want or plan)
+    g = torch.Generator(device=device)
+    g.manual_seed(m + n)
+    x = torch.randn(m, k, generator=g, device=device).to(torch.bfloat16)
+
+    def weights():
+        d = torch.randn(n, k, generator=g, device=device) * 0.05
+        return d.to(torch.bfloat16) if wtype == "bf16" else kernels.quantize(d, wtype)
+
+    w, w_up = weights(), weights()
+    def bound(a):  # two fp32 sums of the same k products, in any order: (k + 8) 2^-24 of their magnitudes each
+        dense = (a if wtype == "bf16" else kernels.dequantize_bf16(a, wtype, k)).double()
+        return 2 * (k + 8) * 2.0 ** -24 * (x.double().abs() @ dense.abs().T)
+
+    if gated:
+        got, one = kernels.gemm_swiglu(x, w, w_up, wtype), kernels.gemm_swiglu(x, w, w_up, wtype, splits=1)
+        if plan[0] == 1:
+            assert torch.equal(got, one)
+        else:  # silu's slope is below 1.1, its value below its argument's; then one bf16 rounding each
+            gate, up = (kernels.gemm(x, a, wtype, out_dtype=torch.float32, splits=1).double().abs() for a in (w, w_up))
+            allowed = 1.1 * bound(w) * (up + bound(w_up)) + gate * bound(w_up)
+            assert ((got.double() - one.double()).abs() <= 2.0 ** -7 * one.double().abs() + allowed).all()
+        return
+    bound = bound(w)
+    res = torch.randn(m, n, generator=g, device=device)
+    one = kernels.gemm(x, w, wtype, out_dtype=torch.float32, splits=1)
+    got = kernels.gemm(x, w, wtype, out_dtype=torch.float32)
+    summed = kernels.gemm(x, w, wtype, out=res.clone(), residual=res)
+    half = kernels.gemm(x, w, wtype)
+    if plan[0] == 1:
+        assert torch.equal(got, one) and torch.equal(half, one.to(torch.bfloat16))
+    assert ((got - one).double().abs() <= bound).all()
+    assert torch.equal(half, got.to(torch.bfloat16))
+    assert ((summed.double() - res.double() - one.double()).abs() <= bound + 2.0 ** -23 * (res.abs() + one.abs())).all()
+    if wtype == "q8_0":
+        bias = torch.randn(n, generator=g, device=device)
+        y = kernels.q8_0_linear(x, w, bias=bias, act="gelu", out_dtype=torch.float32)
+        ref = kernels.q8_0_linear(x, w, bias=bias, act="gelu", out_dtype=torch.float32, splits=1)
+        # gelu's slope is below 1.13; its own fp32 roundings are those of values a few units apart
+        assert ((y - ref).double().abs() <= 1.13 * bound + 2.0 ** -21 * (one.abs() + bias.abs())).all()
+
+
+@pytest.mark.gpu
+def test_planned_linear_keeps_unaligned_rows(device):
+    """Q8_0 rows that start at any even address: not dequantised first (that needs 16 bytes), the same result."""
+    from torch2vk_amd import kernels
+
+    g = torch.Generator(device=device)
+    g.manual_seed(5)
+    m, n, k = 3000, 4100, 2048
+    assert kernels.gemm_plan(m, n, k, "q8_0") == (1, True)
+    x = torch.randn(m, k, generator=g, device=device).to(torch.bfloat16)
+    w = kernels.quantize(torch.randn(n, k, generator=g, device=device) * 0.05, "q8_0")
+    buf = torch.empty(w.numel() + 16, dtype=torch.uint8, device=device)
+    odd = buf[2:2 + w.numel()].view(n, -1)
+    odd.copy_(w)
+    assert torch.equal(kernels.q8_0_linear(x, odd), kernels.q8_0_linear(x, w))

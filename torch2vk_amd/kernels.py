@@ -309,21 +309,24 @@ def lm_head_argmax_partial(x: torch.Tensor, w: torch.Tensor, wtype: str, partial
          ptr(partial_tokens), g, stream_handle())
 
 
-GEMM_FILL_BLOCKS = 128  # grids below this many tiles split K (t2h_gemm_splitk)
-# From this many rows of x, a one-pass prefill GEMM dequantises its packed weights once into a bf16 scratch
-# (t2h_dequantize_bf16, ~1 ns per weight) and runs the tile loop on bf16 rows, instead of dequantising every
-# weight tile once per 256 rows of x inside the loop (measured on MI355X at M 16384, K 4096, N 12288 Q8_0: 1.85 ms
-# in-loop against 0.05 + 1.52 ms; break-even near 2300 rows).  The products are bit-identical either way.
-# 0 disables it.
+GEMM_FILL_BLOCKS = 128  # from DEQUANT_FIRST_ROWS rows, grids below this many tiles split K (t2h_gemm_splitk)
+# From this many rows of x, a one-pass prefill GEMM always dequantises its packed weights once into a bf16 scratch
+# (t2h_dequantize_bf16) and runs the tile loop on bf16 rows, instead of dequantising every weight tile once per 128 or
+# 256 rows of x inside the loop (measured on MI355X at M 16384, K 4096, N 12288 Q8_0: 1.85 ms in-loop against
+# 0.05 + 1.52 ms); below it gemm_plan decides.  The products are bit-identical either way.  0 disables it.
 DEQUANT_FIRST_ROWS = 4096
 
 
-def _dequant_first(m: int, wtype: str, splits: int) -> bool:
-    return DEQUANT_FIRST_ROWS > 0 and m >= DEQUANT_FIRST_ROWS and splits == 1 and wtype != "bf16"
+def _dequantized(wtype: str, k: int, *ws: torch.Tensor) -> list[torch.Tensor] | None:
+    """The weights as bf16 scratch, or None when the device has no room for it: the tile loop takes packed rows too."""
+    try:
+        return [dequantize_bf16(w, wtype, k) for w in ws]
+    except torch.OutOfMemoryError:
+        return None
 
 
 def gemm_splits(m: int, n_cols: int, k: int) -> int:
-    """K parts for a prefill GEMM of m rows and n_cols tile columns (1 = the one-pass GEMM): when the
+    """K parts for a prefill GEMM of many rows and n_cols tile columns (1 = the one-pass GEMM): when the
     one-pass grid has fewer than GEMM_FILL_BLOCKS tiles, enough parts that the split grid (128-row tiles)
     reaches ~256 blocks, each part at least 2 stages of 64, at most 16 parts."""
     tiles_n = -(-n_cols // 256)
@@ -335,7 +338,7 @@ def gemm_splits(m: int, n_cols: int, k: int) -> int:
     return max(1, min(k // 128, -(-256 // split_tiles), 16))
 
 
-GEMM_TILE_MAX_ROWS = 4095  # from 4096 rows a dequantised copy of the weights pays (DEQUANT_FIRST_ROWS)
+GEMM_TILE_MAX_ROWS = 4095  # from 4096 rows a dequantised copy of the weights always pays (DEQUANT_FIRST_ROWS)
 # Tiles of t2h_gemm_tiles by its ``tile`` argument: rows, columns, the longest K taken.
 GEMM_TILES = ((32, 32, 4096), (64, 32, 4096), (64, 64, 6144), (128, 64, 4096))
 
@@ -344,11 +347,11 @@ GEMM_TILES = ((32, 32, 4096), (64, 32, 4096), (64, 64, 6144), (128, 64, 4096))
 def gemm_tile(m: int, n_cols: int, k: int, gated: bool = False) -> int | None:
     """The t2h_gemm_tiles tile for a prefill GEMM of m rows and n_cols tile columns, or None (the 128- and 256-row
     tiles of gemm_q_kernel): the smallest tile whose grid is one block per CU (a block fills a CU's LDS, so a
-    second round costs as much as the first), else 128 x 64 in up to two rounds.  A longer K than the tile's is a
-    serial chain that split-K over idle CUs beats.  Measured (us, tile against split-K or one pass): 128 rows K 1024
+    second round costs as much as the first), else up to K 1024 128 x 64 in up to two rounds.  A longer K than the tile's
+    is a serial chain that split-K over idle CUs beats.  Measured (us, tile against split-K or one pass): 128 rows K 1024
     N 4096, 256 blocks of 64 x 32: 7.4 against 20.7, of 64 x 64 (128 blocks): 9.3; 300 rows: 128 x 64 (192 blocks) 13.6,
     64 x 64 (320) 17.3, split-K 30.6; 520 rows, K 1024 N 2 x 3072: 128 x 64 (480 blocks) 23.6 against 36.3; 1024 rows, the same
-    (768 blocks): 35.3 against 27.5; 627 rows K 4096 N 4096, 320 blocks: 75 against 63; 128 rows K 6144 N 2048: 64 x 32 25.2 against
+    (768 blocks): 35.3 against 27.5; 548 rows K 4096 N 4096, 320 blocks: 66 against 49 in 3 splits; 128 rows K 6144 N 2048: 64 x 32 25.2 against
     22.7; Q6_K K 12288 N 4096: 62 against 47; 22 rows gate|up K 6144 N 2 x 2048, 64 blocks of 64 x 64: 40 against 23.  Over 145 random
     shapes of 9 to 4000 rows the tiles take 0.74 of the time."""
     if m > GEMM_TILE_MAX_ROWS:
@@ -360,9 +363,61 @@ def gemm_tile(m: int, n_cols: int, k: int, gated: bool = False) -> int | None:
         blocks = -(-m // rows) * -(-n_cols // cols)
         if blocks <= 256:
             return tile if k <= (2048 if tile == 2 and blocks < 160 else k_max) else None
-    if k <= 1024 and blocks <= 512 or k <= GEMM_TILES[-1][2] and 448 <= blocks <= 512:
+    if k <= 1024 and blocks <= 512:
         return len(GEMM_TILES) - 1
     return None
+
+
+# What a prefill GEMM below DEQUANT_FIRST_ROWS rows takes, in us: a stage of 64 of K in every CU's 128 x 256 tile by the
+# type of its weight rows (packed ones are converted in the loop; bf16 ones only pass through), a launch, the split
+# products' reduction (a launch, and per MB of them), and t2h_dequantize_bf16 (a launch, and per million weights).
+# Least squares over 1270 timings of 150 random shapes of 150 to 4095 rows, K 1024 to 12288, N 1024 to 2 x 12288.
+_STAGE_US = {"q4_k": 1.36, "q6_k": 1.89, "q8_0": 1.22, "bf16": 0.91}
+_SPLIT_STAGE_US = 1.1  # what the parts are chosen by, whatever the type (0.95 to 1.3 choose alike)
+_LAUNCH_US, _REDUCE_US, _REDUCE_US_MB, _DEQUANT_US, _DEQUANT_US_M = 5.0, 4.0, 0.37, 5.2, 0.64
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_plan(m: int, n: int, k: int, wtype: str, gated: bool = False, dequant: bool = True) -> tuple[int, bool]:
+    """(K parts, whether to dequantise the weights to bf16 first) of a prefill GEMM that gemm_tile gives no tile:
+    the fastest by the figures above.  A tile fills a CU's LDS, so a grid runs in rounds of 256 blocks: a split pays
+    while it fills a round and loses when it starts another, and the in-loop conversion costs in each round what
+    dequantising once costs in one.  Measured (us, before: splits to 256 blocks or more, weights converted in the
+    loop): 1901 rows Q4_K K 4096 gate|up of 12288: 558 -> 403 dequantised; Q6_K K 12288 N 4096: 358 -> 240
+    dequantised; 548 rows Q4_K K 4096 N 4096, 80 tiles: 66 -> 49 in 3 splits (4 start a second round); 735 rows Q6_K,
+    the same, 96 tiles: 106 -> 65 dequantised, in 2.  Over the 150 shapes 0.86 of the time; the best choice for
+    each of them, 0.84."""
+    cols = -(-n * 2 // 256) * 256 if gated else n
+    tiles_n = -(-cols // 256)
+    tiles, tiles_256 = -(-m // 128) * tiles_n, -(-m // 256) * tiles_n
+
+    def us(splits: int, stage: float) -> float:
+        rounds = -(-tiles * splits // 256)
+        if splits == 1 and (tiles_256 >= 1024 or m <= 128):
+            rounds = 2 * -(-tiles_256 // 256)  # 256-row tiles
+        t = _LAUNCH_US + rounds * -(-(k // 64) // splits) * stage
+        return t if splits == 1 else t + _REDUCE_US + _REDUCE_US_MB * splits * m * cols * 4e-6
+
+    parts = [1] + [s for s in range(2, min(k // 128, 16) + 1) if tiles * s <= 512]
+    # the same parts for every type, so that packed rows and their bf16 copy give the same sums
+    splits = min(parts, key=lambda s: us(s, _SPLIT_STAGE_US))
+    if not dequant or wtype == "bf16":
+        return splits, False
+    once = (2 if gated else 1) * (_DEQUANT_US + _DEQUANT_US_M * n * k * 1e-6)
+    # a scratch of the weights' size is not taken for a tie
+    return splits, us(splits, _STAGE_US["bf16"]) + once < 0.92 * us(splits, _STAGE_US[wtype])
+
+
+def _gemm_plan(m: int, n: int, k: int, wtype: str, splits: int | None, gated: bool = False,
+               dequant: bool = True) -> tuple[int, bool]:
+    """(K parts, dequantise first): as the caller gave the parts, by gemm_plan, or from DEQUANT_FIRST_ROWS rows by
+    gemm_splits."""
+    dequant = dequant and DEQUANT_FIRST_ROWS > 0 and wtype != "bf16"
+    if splits is None and m <= GEMM_TILE_MAX_ROWS:
+        return gemm_plan(m, n, k, wtype, gated, dequant)
+    if splits is None:
+        splits = gemm_splits(m, 2 * n if gated else n, k)
+    return splits, dequant and m >= DEQUANT_FIRST_ROWS and splits == 1
 
 
 def _gemm_tiles(wtype: str, x: torch.Tensor, w: torch.Tensor, w_up: torch.Tensor | None, out: torch.Tensor, m: int,
@@ -386,7 +441,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor | No
          splits: int | None = None) -> torch.Tensor:
     """Prefill GEMM on the matrix cores: y[M, N] = x[M, K] . deq(W)^T (+ residual); x bf16, W Q8_0, Q4_K or
     Q6_K packed rows, or bf16 [N, K] ("bf16", e.g. from :func:`dequantize_bf16`).  ``splits``: K parts
-    (t2h_gemm_splitk; None = gemm_tile's choice of small tiles, else gemm_splits'; 1 = one pass)."""
+    (t2h_gemm_splitk; None = gemm_tile's choice of small tiles, else gemm_plan's; 1 = one pass)."""
     if wtype not in ("q8_0", "q4_k", "q6_k", "bf16"):
         raise ValueError(f"gemm handles q8_0, q4_k, q6_k and bf16 weights, got {wtype!r}")
     _check(x, "x", torch.bfloat16)
@@ -409,12 +464,13 @@ def gemm(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor | No
         if tile is not None:
             _gemm_tiles(wtype, x, w, None, out, m, k, n, k, tile, residual=residual)
             return out
-        splits = gemm_splits(m, n, k)
+    splits, dequant = _gemm_plan(m, n, k, wtype, splits)
+    dense = _dequantized(wtype, k, w) if dequant else None
+    if dense is not None:
+        (w,), wtype = dense, "bf16"
     if splits > 1:
         _gemm_splitk(wtype, x, w, None, out, m, k, n, k, splits, residual=residual)
         return out
-    if _dequant_first(m, wtype, splits):
-        w, wtype = dequantize_bf16(w, wtype, k), "bf16"
     name = {"q8_0": "t2h_q8_0_gemm", "q4_k": "t2h_q4k_gemm", "q6_k": "t2h_q6k_gemm", "bf16": "t2h_bf16_gemm"}[wtype]
     call(name, ptr(x), ptr(w), ptr(out), _OUT_DTYPES[out.dtype], ptr(residual), m, k, n, stream_handle())
     return out
@@ -445,12 +501,13 @@ def gemm_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, wtype
         if tile is not None:
             _gemm_tiles(wtype, x, w_gate, w_up, out, m, k, n, k, tile)
             return out
-        splits = gemm_splits(m, 2 * n, k)
+    splits, dequant = _gemm_plan(m, n, k, wtype, splits, gated=True)
+    dense = _dequantized(wtype, k, w_gate, w_up) if dequant else None
+    if dense is not None:
+        (w_gate, w_up), wtype = dense, "bf16"
     if splits > 1:
         _gemm_splitk(wtype, x, w_gate, w_up, out, m, k, n, k, splits)
         return out
-    if _dequant_first(m, wtype, splits):
-        w_gate, w_up, wtype = dequantize_bf16(w_gate, wtype, k), dequantize_bf16(w_up, wtype, k), "bf16"
     call("t2h_gemm_swiglu", WTYPES[wtype], ptr(x), ptr(w_gate), ptr(w_up), ptr(out), m, k, n, stream_handle())
     return out
 
@@ -564,8 +621,8 @@ def q8_0_linear(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None =
     """y[M, N] = act(x[M, K] . deq(W)^T + bias) (+ residual) on the matrix cores (LINEAR_BIAS_Q8_0W_F32B_F32).
     x bf16 with K % 64 == 0; W Q8_0 rows of w_k = 32 * blocks <= K values (x's columns past w_k must be
     finite: they multiply zeros); bias fp32 [N]; act None or "gelu" (erf by Abramowitz-Stegun 7.1.26, as the
-    reference).  From DEQUANT_FIRST_ROWS rows with w_k == K, W is dequantised once and the bf16 rows run
-    t2h_bf16_linear (the same bits)."""
+    reference).  Where gemm_plan or DEQUANT_FIRST_ROWS says so, with w_k == K and 16-byte aligned rows, W is
+    dequantised once and the bf16 rows run t2h_bf16_linear (the same products)."""
     _check(x, "x", torch.bfloat16)
     _check(w, "weight", torch.uint8, align=1)
     k = int(x.shape[-1])
@@ -600,17 +657,18 @@ def q8_0_linear(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None =
         if tile is not None:
             _gemm_tiles("q8_0", x, w, None, out, m, k, n, w_k, tile, bias=bias, act=ACTS[act], residual=residual)
             return out
-        splits = gemm_splits(m, n, k)
+    splits, dequant = _gemm_plan(m, n, k, "q8_0", splits, dequant=w_k == k and w.data_ptr() % 16 == 0)
+    dense, wtype = _dequantized("q8_0", k, w) if dequant else None, "q8_0"
+    if dense is not None:
+        (w,), wtype = dense, "bf16"
     if splits > 1:
-        _gemm_splitk("q8_0", x, w, None, out, m, k, n, w_k, splits, bias=bias, act=ACTS[act], residual=residual)
-        return out
-    if w_k == k and _dequant_first(m, "q8_0", splits):
-        wb = dequantize_bf16(w, "q8_0", k)
-        call("t2h_bf16_linear", ptr(x), ptr(wb), ptr(bias), ACTS[act], ptr(out), _OUT_DTYPES[out.dtype], ptr(residual),
+        _gemm_splitk(wtype, x, w, None, out, m, k, n, w_k, splits, bias=bias, act=ACTS[act], residual=residual)
+    elif wtype == "bf16":
+        call("t2h_bf16_linear", ptr(x), ptr(w), ptr(bias), ACTS[act], ptr(out), _OUT_DTYPES[out.dtype], ptr(residual),
              m, k, n, stream_handle())
-        return out
-    call("t2h_q8_0_linear", ptr(x), ptr(w), ptr(bias), ACTS[act], ptr(out), _OUT_DTYPES[out.dtype], ptr(residual),
-         m, k, n, w_k, stream_handle())
+    else:
+        call("t2h_q8_0_linear", ptr(x), ptr(w), ptr(bias), ACTS[act], ptr(out), _OUT_DTYPES[out.dtype], ptr(residual),
+             m, k, n, w_k, stream_handle())
     return out
 
 
