@@ -30,22 +30,18 @@ __device__ __forceinline__ float round_away(float value) {
     return s * rounded;
 }
 
-// block = 64 threads = two Q8_0 blocks; grid.x over (rows * blocks_per_row / 2)
-__global__ __launch_bounds__(64) void quantize_q8_0_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
-                                                           uint32_t k, uint64_t total_blocks) {
-    const uint64_t blk = (uint64_t)blockIdx.x * 2 + (threadIdx.x >> 5);
+// block = 256 threads = eight Q8_0 blocks, one lane a value.  Rows are whole blocks, so block i starts at value 32 i.
+// The largest magnitude is the same in any order: five exchanges.  Reading every value lane by lane, in blocks of one
+// wave, was most of the kernel's time (4096 x 4096: 94 us; now 44).
+__global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
+                                                            uint64_t total_blocks) {
+    const uint64_t blk = (uint64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
     const int lane = threadIdx.x & 31;
     if (blk >= total_blocks) return;
-    const uint32_t bpr = k / 32;
-    const uint64_t row = blk / bpr;
-    const uint64_t b = blk % bpr;
-    const float value = x[row * k + b * 32 + lane];
-    float amax = 0.0f;
-    // sequential max in index order, as the reference's lane 0 does
-    for (int i = 0; i < 32; ++i) {
-        const float vi = __shfl(value, (threadIdx.x & 32) + i, 64);
-        amax = fmaxf(amax, fabsf(vi));
-    }
+    const float value = x[blk * 32 + lane];
+    float amax = fmaxf(0.0f, fabsf(value));
+#pragma unroll
+    for (int d = 16; d; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d, 64));
     const float block_scale = amax / 127.0f;
     const float inv_scale = block_scale == 0.0f ? 0.0f : 1.0f / block_scale;
     int quant = (int)round_away(value * inv_scale);
@@ -65,29 +61,33 @@ __device__ __forceinline__ uint32_t rounded_code(float value, uint32_t max_code)
     return (uint32_t)clampf_(floorf(value + 0.5f), 0.0f, (float)max_code);
 }
 
-__device__ float weighted_quant_error(const float* v, float scale, float minimum, float inv_scale) {
+// the code as a float: it is whole already, and NaN gives 0 as the conversion does
+__device__ __forceinline__ float rounded_level(float value) { return clampf_(floorf(value + 0.5f), 0.0f, 15.0f); }
+
+__device__ __forceinline__ float weighted_quant_error(const float (&v)[32], const float (&weight)[32], float scale,
+                                                      float minimum, float inv_scale) {
     float error = 0.0f;
-    float sum_x2 = 0.0f;
+#pragma unroll
     for (int i = 0; i < 32; ++i) {
-        const float t = v[i] * v[i];
-        sum_x2 = sum_x2 + t;
-    }
-    const float av_x = sqrtf(sum_x2 / 32.0f);
-    for (int i = 0; i < 32; ++i) {
-        const float weight = av_x + fabsf(v[i]);
-        const float level = (float)rounded_code(inv_scale * (v[i] - minimum), 15u);
+        const float level = rounded_level(inv_scale * (v[i] - minimum));
         const float sl = scale * level;
         const float diff = (sl + minimum) - v[i];
-        const float wd = weight * diff;
+        const float wd = weight[i] * diff;
         error = error + wd * diff;
     }
     return error;
 }
 
-__device__ float choose_subblock_scale(const float* v, float* min_offset) {
+// The search over 21 scales is all of the kernel's time, and VALU instructions are all of the search's: 21 sums of 32
+// serial terms twice.  The values, their weights and their distances from the minimum stay in registers under
+// constant indices (a loop of four indexed them at run time, two scalar instructions and a move a value), which
+// leaves 21 instructions a value and scale of 31.  4096 x 4096: 238 -> 174 us at 144 registers; held to 128 of them,
+// 16 spill: 187.
+__device__ __forceinline__ float choose_subblock_scale(const float (&v)[32], float* min_offset) {
     float min_value = v[0];
     float max_value = v[0];
     float sum_x2 = 0.0f;
+#pragma unroll
     for (int i = 0; i < 32; ++i) {
         min_value = fminf(min_value, v[i]);
         max_value = fmaxf(max_value, v[i]);
@@ -100,26 +100,30 @@ __device__ float choose_subblock_scale(const float* v, float* min_offset) {
         return 0.0f;
     }
     const float av_x = sqrtf(sum_x2 / 32.0f);
+    float weight[32], above[32];
     float sum_w = 0.0f;
     float sum_x = 0.0f;
+#pragma unroll
     for (int i = 0; i < 32; ++i) {
-        const float weight = av_x + fabsf(v[i]);
-        sum_w = sum_w + weight;
-        const float wx = weight * v[i];
+        weight[i] = av_x + fabsf(v[i]);
+        above[i] = v[i] - min_value;
+        sum_w = sum_w + weight[i];
+        const float wx = weight[i] * v[i];
         sum_x = sum_x + wx;
     }
     float inv_scale = 15.0f / (max_value - min_value);
     float best_scale = 1.0f / inv_scale;
     float best_min = min_value;
-    float best_error = weighted_quant_error(v, best_scale, best_min, inv_scale);
+    float best_error = weighted_quant_error(v, weight, best_scale, best_min, inv_scale);
+#pragma unroll 1
     for (uint32_t step = 0; step <= 20u; ++step) {
         const float stepped = 0.1f * (float)step;
         inv_scale = (14.0f + stepped) / (max_value - min_value);
         float sum_l = 0.0f, sum_l2 = 0.0f, sum_xl = 0.0f;
+#pragma unroll
         for (int i = 0; i < 32; ++i) {
-            const float weight = av_x + fabsf(v[i]);
-            const float level = (float)rounded_code(inv_scale * (v[i] - min_value), 15u);
-            const float wl = weight * level;
+            const float level = rounded_level(inv_scale * above[i]);
+            const float wl = weight[i] * level;
             sum_l = sum_l + wl;
             const float wll = wl * level;
             sum_l2 = sum_l2 + wll;
@@ -140,7 +144,7 @@ __device__ float choose_subblock_scale(const float* v, float* min_offset) {
                 candidate_min = 0.0f;
                 candidate_scale = sum_l2 > 0.0f ? sum_xl / sum_l2 : 0.0f;
             }
-            const float candidate_error = weighted_quant_error(v, candidate_scale, candidate_min, inv_scale);
+            const float candidate_error = weighted_quant_error(v, weight, candidate_scale, candidate_min, inv_scale);
             if (candidate_error < best_error) {
                 best_error = candidate_error;
                 best_scale = candidate_scale;
@@ -152,18 +156,16 @@ __device__ float choose_subblock_scale(const float* v, float* min_offset) {
     return fmaxf(0.0f, best_scale);
 }
 
-// block = 64 threads = 8 superblocks, 8 lanes (one sub-block each) per superblock
+// block = 64 threads = 8 superblocks, 8 lanes (one sub-block each) per superblock; superblock i starts at value 256 i
 __global__ __launch_bounds__(64) void quantize_q4_k_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
-                                                           uint32_t k, uint64_t total_blocks) {
+                                                           uint64_t total_blocks) {
     const uint64_t blk = (uint64_t)blockIdx.x * 8 + (threadIdx.x >> 3);
     const int sub = threadIdx.x & 7;
     const int group_base = threadIdx.x & ~7;
     if (blk >= total_blocks) return;
-    const uint32_t bpr = k / 256;
-    const uint64_t row = blk / bpr;
-    const uint64_t b = blk % bpr;
-    const float* src = x + row * k + b * 256 + sub * 32;
+    const float* src = x + blk * 256 + sub * 32;
     float v[32];
+#pragma unroll
     for (int i = 0; i < 32; ++i) v[i] = src[i];
 
     float min_offset = 0.0f;
@@ -172,6 +174,7 @@ __global__ __launch_bounds__(64) void quantize_q4_k_kernel(const float* __restri
     // lane 0 of the superblock's semantics: sequential max over sub-blocks 0..7
     float max_scale = 0.0f, max_min = 0.0f;
     float scales[8], mins[8];
+#pragma unroll
     for (int j = 0; j < 8; ++j) {
         scales[j] = __shfl(sscale, group_base + j, 64);
         mins[j] = __shfl(min_offset, group_base + j, 64);
@@ -183,6 +186,7 @@ __global__ __launch_bounds__(64) void quantize_q4_k_kernel(const float* __restri
     const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
     const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
     uint32_t scale_codes[8], min_codes[8];
+#pragma unroll
     for (int j = 0; j < 8; ++j) {
         scale_codes[j] = rounded_code(scales[j] * inv_scale, 63u);
         min_codes[j] = rounded_code(mins[j] * inv_min, 63u);
@@ -190,13 +194,14 @@ __global__ __launch_bounds__(64) void quantize_q4_k_kernel(const float* __restri
     d_scale = round_f16(d_scale);
     d_min = round_f16(d_min);
 
-    const float scale = d_scale * (float)scale_codes[sub];
-    const float minimum = d_min * (float)min_codes[sub];
-    uint32_t quants[32];
+    const float scale = d_scale * (float)rounded_code(sscale * inv_scale, 63u);
+    const float minimum = d_min * (float)rounded_code(min_offset * inv_min, 63u);
+    uint32_t quants[8];  // four codes a word
+#pragma unroll
     for (int i = 0; i < 32; ++i) {
         uint32_t q = 0u;
         if (scale > 0.0f) q = rounded_code((v[i] + minimum) / scale, 15u);
-        quants[i] = q;
+        quants[i / 4] = i % 4 ? quants[i / 4] | (q << (8 * (i % 4))) : q;
     }
     uint8_t* o = out + blk * 144;
     if (sub == 0) {
@@ -215,11 +220,15 @@ __global__ __launch_bounds__(64) void quantize_q4_k_kernel(const float* __restri
     // sub-block s lives in nibble group s/2: low nibbles if s even, high if odd
     const int group = sub >> 1;
     const bool high = (sub & 1) != 0;
-    // combine with the partner lane's nibbles so each byte is written once
-    for (int i = 0; i < 32; ++i) {
-        const uint32_t partner = (uint32_t)__shfl((int)quants[i], threadIdx.x ^ 1, 64);
-        if (!high) o[16 + group * 32 + i] = (uint8_t)((quants[i] & 15u) | ((partner & 15u) << 4));
+    // combine with the partner lane's nibbles, each lane of the pair storing half of the group's 32 bytes
+    uint32_t words[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t send = high ? quants[i] : quants[4 + i], keep = high ? quants[4 + i] : quants[i];
+        const uint32_t partner = (uint32_t)__shfl_xor((int)send, 1, 64);
+        words[i] = high ? partner | (keep << 4) : keep | (partner << 4);
     }
+    __builtin_memcpy(o + 16 + group * 32 + (high ? 16 : 0), words, 16);  // out has any alignment
 }
 
 // ------------------------------------------------------------------ Q6_K --
@@ -227,8 +236,9 @@ __global__ __launch_bounds__(64) void quantize_q4_k_kernel(const float* __restri
 __device__ __forceinline__ int nearest_int(float value) { return (int)rintf(value); }
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-__device__ float make_qx_quants16(const float* v, int* levels) {
+__device__ __forceinline__ float make_qx_quants16(const float (&v)[16], int (&levels)[16]) {
     float max_value = 0.0f, max_abs = 0.0f;
+#pragma unroll
     for (int i = 0; i < 16; ++i) {
         const float a = fabsf(v[i]);
         if (a > max_abs) {
@@ -237,67 +247,70 @@ __device__ float make_qx_quants16(const float* v, int* levels) {
         }
     }
     if (max_abs < 1.0e-12f) {
+#pragma unroll
         for (int i = 0; i < 16; ++i) levels[i] = 32;
         return 0.0f;
     }
-    float inv_scale = -32.0f / max_value;
-    float sum_lx = 0.0f, sum_l2 = 0.0f;
+    // as in Q4_K's search: products that no scale changes are made once (4096 x 4096: 134 -> 100 us)
+    float weight[16], wv[16];
+#pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const int level = clampi(nearest_int(inv_scale * v[i]), -32, 31);
-        levels[i] = level + 32;
-        const float weight = v[i] * v[i];
-        const float wv = weight * v[i];
-        const float wvl = wv * (float)level;
-        sum_lx = sum_lx + wvl;
-        const float wll = weight * (float)(level * level);
-        sum_l2 = sum_l2 + wll;
+        weight[i] = v[i] * v[i];
+        wv[i] = weight[i] * v[i];
     }
+    // the sums of one scale; a level's square is whole and below 2^11, so its float product is exact
+    const auto sums = [&](float inv_scale, float& sum_lx, float& sum_l2) {
+        sum_lx = 0.0f;
+        sum_l2 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float level = (float)clampi(nearest_int(inv_scale * v[i]), -32, 31);
+            const float wvl = wv[i] * level;
+            sum_lx = sum_lx + wvl;
+            const float wll = weight[i] * (level * level);
+            sum_l2 = sum_l2 + wll;
+        }
+    };
+    float best_inv = -32.0f / max_value;
+    float sum_lx, sum_l2;
+    sums(best_inv, sum_lx, sum_l2);
     float scale = sum_l2 > 0.0f ? sum_lx / sum_l2 : 0.0f;
     float best = scale * sum_lx;
+#pragma unroll 1
     for (int step = -9; step <= 9; ++step) {
         if (step == 0) continue;
         const float stepped = 0.1f * (float)step;
         const float numer = 32.0f + stepped;
-        inv_scale = -numer / max_value;
-        sum_lx = 0.0f;
-        sum_l2 = 0.0f;
-        for (int i = 0; i < 16; ++i) {
-            const int level = clampi(nearest_int(inv_scale * v[i]), -32, 31);
-            const float weight = v[i] * v[i];
-            const float wv = weight * v[i];
-            const float wvl = wv * (float)level;
-            sum_lx = sum_lx + wvl;
-            const float wll = weight * (float)(level * level);
-            sum_l2 = sum_l2 + wll;
-        }
+        const float inv_scale = -numer / max_value;
+        sums(inv_scale, sum_lx, sum_l2);
         const float lhs = sum_lx * sum_lx;
         const float rhs = best * sum_l2;
         if (sum_l2 > 0.0f && lhs > rhs) {
-            for (int i = 0; i < 16; ++i) levels[i] = clampi(nearest_int(inv_scale * v[i]), -32, 31) + 32;
+            best_inv = inv_scale;
             scale = sum_lx / sum_l2;
             best = scale * sum_lx;
         }
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) levels[i] = clampi(nearest_int(best_inv * v[i]), -32, 31) + 32;
     return scale;
 }
 
 // block = 64 threads = 4 superblocks, 16 lanes (one 16-value sub-block each) per superblock
 __global__ __launch_bounds__(64) void quantize_q6_k_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
-                                                           uint32_t k, uint64_t total_blocks) {
+                                                           uint64_t total_blocks) {
     __shared__ int lv[4][256];
     const int sbk = threadIdx.x >> 4;
     const uint64_t blk = (uint64_t)blockIdx.x * 4 + sbk;
     const int sub = threadIdx.x & 15;
     const int group_base = threadIdx.x & ~15;
     const bool active = blk < total_blocks;
-    const uint32_t bpr = k / 256;
     float v[16];
     int levels[16];
     float bscale = 0.0f;
     if (active) {
-        const uint64_t row = blk / bpr;
-        const uint64_t b = blk % bpr;
-        const float* src = x + row * k + b * 256 + sub * 16;
+        const float* src = x + blk * 256 + sub * 16;
+#pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = src[i];
         bscale = make_qx_quants16(v, levels);
     }
@@ -442,10 +455,10 @@ extern "C" int t2h_quantize_q8_0(const float* x, uint32_t rows, uint32_t k, void
     int st = quant_check(x, out, rows, k, 32);
     if (st) return st;
     const uint64_t total = (uint64_t)rows * (k / 32);
-    const uint64_t grid = (total + 1) / 2;
-    if (grid > 0x7fffffffull) return T2H_ERR_SHAPE;
-    hipLaunchKernelGGL(quantize_q8_0_kernel, dim3((uint32_t)grid), dim3(64), 0, (hipStream_t)stream, x,
-                       (uint8_t*)out, k, total);
+    const uint64_t grid = (total + 7) / 8;
+    if ((total + 1) / 2 > 0x7fffffffull) return T2H_ERR_SHAPE;
+    hipLaunchKernelGGL(quantize_q8_0_kernel, dim3((uint32_t)grid), dim3(256), 0, (hipStream_t)stream, x,
+                       (uint8_t*)out, total);
     T2H_LAUNCH_CHECK();
     return T2H_OK;
 }
@@ -457,7 +470,7 @@ extern "C" int t2h_quantize_q4_k(const float* x, uint32_t rows, uint32_t k, void
     const uint64_t grid = (total + 7) / 8;
     if (grid > 0x7fffffffull) return T2H_ERR_SHAPE;
     hipLaunchKernelGGL(quantize_q4_k_kernel, dim3((uint32_t)grid), dim3(64), 0, (hipStream_t)stream, x,
-                       (uint8_t*)out, k, total);
+                       (uint8_t*)out, total);
     T2H_LAUNCH_CHECK();
     return T2H_OK;
 }
@@ -469,7 +482,7 @@ extern "C" int t2h_quantize_q6_k(const float* x, uint32_t rows, uint32_t k, void
     const uint64_t grid = (total + 3) / 4;
     if (grid > 0x7fffffffull) return T2H_ERR_SHAPE;
     hipLaunchKernelGGL(quantize_q6_k_kernel, dim3((uint32_t)grid), dim3(64), 0, (hipStream_t)stream, x,
-                       (uint8_t*)out, k, total);
+                       (uint8_t*)out, total);
     T2H_LAUNCH_CHECK();
     return T2H_OK;
 }
