@@ -371,10 +371,11 @@ def gemm_tile(m: int, n_cols: int, k: int, gated: bool = False) -> int | None:
 # What a prefill GEMM below DEQUANT_FIRST_ROWS rows takes, in us: a stage of 64 of K in every CU's 128 x 256 tile by the
 # type of its weight rows (packed ones are converted in the loop; bf16 ones only pass through), a launch, the split
 # products' reduction (a launch, and per MB of them), and t2h_dequantize_bf16 (a launch, and per million weights).
-# Least squares over 1270 timings of 150 random shapes of 150 to 4095 rows, K 1024 to 12288, N 1024 to 2 x 12288.
+# Least squares over 1270 timings of 150 random shapes of 150 to 4095 rows, K 1024 to 12288, N 1024 to 2 x 12288 (the
+# dequantisation's launch is what a short one costs the host).
 _STAGE_US = {"q4_k": 1.36, "q6_k": 1.89, "q8_0": 1.22, "bf16": 0.91}
 _SPLIT_STAGE_US = 1.1  # what the parts are chosen by, whatever the type (0.95 to 1.3 choose alike)
-_LAUNCH_US, _REDUCE_US, _REDUCE_US_MB, _DEQUANT_US, _DEQUANT_US_M = 5.0, 4.0, 0.37, 5.2, 0.64
+_LAUNCH_US, _REDUCE_US, _REDUCE_US_MB, _DEQUANT_US, _DEQUANT_US_M = 5.0, 4.0, 0.37, 5.2, 0.40
 
 
 @functools.lru_cache(maxsize=4096)
@@ -383,10 +384,9 @@ def gemm_plan(m: int, n: int, k: int, wtype: str, gated: bool = False, dequant: 
     the fastest by the figures above.  A tile fills a CU's LDS, so a grid runs in rounds of 256 blocks: a split pays
     while it fills a round and loses when it starts another, and the in-loop conversion costs in each round what
     dequantising once costs in one.  Measured (us, before: splits to 256 blocks or more, weights converted in the
-    loop): 1901 rows Q4_K K 4096 gate|up of 12288: 558 -> 403 dequantised; Q6_K K 12288 N 4096: 358 -> 240
+    loop): 1901 rows Q4_K K 4096 gate|up of 12288: 558 -> 368 dequantised; Q6_K K 12288 N 4096: 358 -> 224
     dequantised; 548 rows Q4_K K 4096 N 4096, 80 tiles: 66 -> 49 in 3 splits (4 start a second round); 735 rows Q6_K,
-    the same, 96 tiles: 106 -> 65 dequantised, in 2.  Over the 150 shapes 0.86 of the time; the best choice for
-    each of them, 0.84."""
+    the same, 96 tiles: 106 -> 60 dequantised, in 2.  Over 85 other random shapes within 1.5 % of the best choice for each."""
     cols = -(-n * 2 // 256) * 256 if gated else n
     tiles_n = -(-cols // 256)
     tiles, tiles_256 = -(-m // 128) * tiles_n, -(-m // 256) * tiles_n
@@ -405,7 +405,7 @@ def gemm_plan(m: int, n: int, k: int, wtype: str, gated: bool = False, dequant: 
         return splits, False
     once = (2 if gated else 1) * (_DEQUANT_US + _DEQUANT_US_M * n * k * 1e-6)
     # a scratch of the weights' size is not taken for a tie
-    return splits, us(splits, _STAGE_US["bf16"]) + once < 0.92 * us(splits, _STAGE_US[wtype])
+    return splits, us(splits, _STAGE_US["bf16"]) + once < 0.95 * us(splits, _STAGE_US[wtype])
 
 
 def _gemm_plan(m: int, n: int, k: int, wtype: str, splits: int | None, gated: bool = False,
