@@ -228,18 +228,19 @@ __global__ __launch_bounds__(WPB * 64) void q4k_gemv_kernel(const Q4GemvArgs a) 
     float best_score = -3.4028234663852886e38f;
     uint32_t best_token = 0xffffffffu;
 
+    const size_t token0 = (size_t)blockIdx.y * a.parts[0].n;  // token blockIdx.y's first output (one part then)
     auto store_row = [&](uint32_t row, float v) {
         int pi = 0;
         pi += (a.n_parts > 1 && row >= a.parts[1].row_begin) ? 1 : 0;
         pi += (a.n_parts > 2 && row >= a.parts[2].row_begin) ? 1 : 0;
         const Q4Part& p = a.parts[pi];
-        const size_t local = (size_t)blockIdx.y * p.n + (row - p.row_begin);  // token blockIdx.y (one part then)
+        const uint32_t local = row - p.row_begin;
         if constexpr (EPI == Q4EPI_F32) {
-            reinterpret_cast<float*>(p.y)[local] = v;
+            (reinterpret_cast<float*>(p.y) + token0)[local] = v;
         } else if constexpr (EPI == Q4EPI_BF16) {
-            reinterpret_cast<uint16_t*>(p.y)[local] = (uint16_t)f32_to_bf16_bits(v);
+            (reinterpret_cast<uint16_t*>(p.y) + token0)[local] = (uint16_t)f32_to_bf16_bits(v);
         } else if constexpr (EPI == Q4EPI_RESID) {
-            reinterpret_cast<float*>(p.y)[local] = a.residual[local] + v;
+            (reinterpret_cast<float*>(p.y) + token0)[local] = (a.residual + token0)[local] + v;
         }
     };
 

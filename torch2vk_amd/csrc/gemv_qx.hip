@@ -237,6 +237,7 @@ __global__ __launch_bounds__(QX_THREADS) void qx_gemv_kernel(const QxArgs a) {
     __syncthreads();
 
     // --------------------------------------------------------- pieces -----
+    const size_t token0 = (size_t)blockIdx.y * (a.n_units * RPW);  // token blockIdx.y's first output
     const uint32_t P = a.pieces;
     int rloc[NIT], sub[NIT], e0[NIT];
     uint32_t woff[NIT];
@@ -300,13 +301,13 @@ __global__ __launch_bounds__(QX_THREADS) void qx_gemv_kernel(const QxArgs a) {
             float v = res[0];
 #pragma unroll
             for (int r = 1; r < RPW; ++r) v = (lane == r) ? res[r] : v;
-            const size_t row = (size_t)blockIdx.y * (a.n_units * RPW) + (row0 + lane);  // token blockIdx.y
+            const uint32_t row = row0 + lane;
             if constexpr (EPI == QXEPI_F32) {
-                reinterpret_cast<float*>(a.y)[row] = v;
+                (reinterpret_cast<float*>(a.y) + token0)[row] = v;
             } else if constexpr (EPI == QXEPI_BF16) {
-                reinterpret_cast<uint16_t*>(a.y)[row] = (uint16_t)f32_to_bf16_bits(v);
+                (reinterpret_cast<uint16_t*>(a.y) + token0)[row] = (uint16_t)f32_to_bf16_bits(v);
             } else if constexpr (EPI == QXEPI_RESID) {
-                reinterpret_cast<float*>(a.y)[row] = a.residual[row] + v;
+                (reinterpret_cast<float*>(a.y) + token0)[row] = (a.residual + token0)[row] + v;
             }
         }
     };
