@@ -457,8 +457,8 @@ int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_strides, const vo
 
 /* The audio codec's whole decoder (run_audio_decode, src/models/quantized_omnivoice/dispatch/audio_decode.py:
  * 60-760) enqueued as one chain of fused launches: codes int64 [codebooks, frames] -> waveform fp32 [frames times the
- * strides' product].  dims: codebooks (<= 32), vocab, codebook_dim, latent, hidden, channels, blocks (<= 16), then
- * each block's stride (transposed conv of kernel 2 stride, padding ceil(stride / 2), output padding stride % 2);
+ * strides' product].  dims: codebooks (<= 32), codebook_dim, latent, hidden, channels, blocks (<= 16), then each
+ * block's stride (transposed conv of kernel 2 stride, padding ceil(stride / 2), output padding stride % 2);
  * every channel count % 8 == 0, channels halved by each block.  ptrs (codebooks + 9 + 21 blocks, in this order):
  * each codebook's Q8_0 table; project_out of all codebooks side by side (fragments, columns c dim + i), the sum of
  * its biases; fc2 (fragments), bias; conv1 (fragments, 7 taps), bias; block 0's alpha; per block: the transposed
@@ -466,7 +466,8 @@ int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_strides, const vo
  * alpha, second conv (fragments, 1 tap), bias, the alpha that follows (next unit, next block, or the last one);
  * then conv2 (fragments, 7 taps, one column), bias.  Fragments: bf16 [tap][step of 16 inputs][tile of 32
  * columns][64][8], lane l holding column l % 32 and inputs 8 (l / 32) .. + 7, inputs padded with zeros to 32 and
- * columns to 64.  Rounding as in the operators one by one: convolution weights and inputs bf16, the rest fp32.
+ * columns to 64.  table_rows: the rows of each codebook's table (a code outside its table embeds as zeros).
+ * Rounding as in the operators one by one: convolution weights and inputs bf16, the rest fp32.
  * stages (or NULL): 1 + 4 blocks fp32 buffers for the activation after conv1, and after each block's transposed
  * conv and residual units.  workspace: t2h_codec_decode_workspace_bytes (0: dims or frames not supported), 256-byte
  * aligned. */
@@ -476,9 +477,9 @@ size_t t2h_codec_decode_workspace_bytes(const uint32_t* dims, uint32_t frames);
  * matrices side by side: cin % 32 == 0 for all but the last).  Each weight d q rounded once to bf16. */
 int t2h_conv_fragments_q8_0(const void* w, uint32_t n, uint32_t cin, uint32_t taps, uint32_t ksteps, uint32_t kstep0,
                             void* out, void* stream);
-int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, uint32_t n_ptrs, const int64_t* codes,
-                     uint32_t frames, float eps, float* out, float* const* stages, void* workspace,
-                     size_t workspace_bytes, void* stream);
+int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, uint32_t n_ptrs, const uint32_t* table_rows,
+                     const int64_t* codes, uint32_t frames, float eps, float* out, float* const* stages,
+                     void* workspace, size_t workspace_bytes, void* stream);
 
 /* ----------------------------------------------- OmniVoice token loop --- */
 /* hidden fp32 [B, S, H] = sum over c < C of audio_w row (c * V + ids[b, c, s]) where audio_mask[b, s] != 0,

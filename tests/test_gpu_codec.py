@@ -95,3 +95,35 @@ def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, ch
     for what, a, b in checks:
         assert a.shape == b.shape, what
         assert_close(a, b, max_abs=2.0 ** -8 * float(np.abs(b).max()), min_cos=0.99999, what=what)
+
+
+def _small_codec(device, seed, **fields):
+    """A decoder whose shapes the fused chain takes, its dense weights, and codes of one id past its vocab."""
+    from torch2vk_amd.omnivoice.decoder import AudioDecoderConfig, OmniVoiceAudioDecoder, synthetic_dense
+
+    cfg = AudioDecoderConfig(**{**dict(codebooks=2, vocab=16, codebook_dim=32, latent=64, hidden=64, channels=64,
+                                       strides=(3, 2)), **fields})
+    dense = synthetic_dense(cfg, seed=seed)
+    codes = torch.from_numpy(np.random.default_rng(seed).integers(0, cfg.vocab + 1, (cfg.codebooks, 9)))
+    codes[0, 0] = cfg.vocab
+    return OmniVoiceAudioDecoder(cfg, dense, device), cfg, dense, codes
+
+
+@pytest.mark.parametrize("extra", [1, -5])
+def test_codec_tables_have_their_own_row_counts(device, extra):
+    """A codebook with more rows than cfg.vocab (a mask row) is looked up by its own row count, and ids past a shorter
+    one embed as zeros: the same samples as with a table padded with zeros to the ids used."""
+    from torch2vk_amd.omnivoice.decoder import OmniVoiceAudioDecoder
+
+    dec, cfg, dense, codes = _small_codec(device, 11)
+    rng = np.random.default_rng(12)
+    rows = cfg.vocab + extra
+    tables = {n: (rng.standard_normal((rows, cfg.codebook_dim)) * 0.2).astype(np.float32)
+              for n in dense if n.startswith("cb")}
+    full = {n: np.concatenate([t, np.zeros((max(0, cfg.vocab + 1 - rows), cfg.codebook_dim), np.float32)])
+            for n, t in tables.items()}
+    got = OmniVoiceAudioDecoder(cfg, {**dense, **tables}, device).decode(codes)
+    want = OmniVoiceAudioDecoder(type(cfg)(**{**vars(cfg), "vocab": cfg.vocab + 1}), {**dense, **full}, device)
+    assert torch.equal(got, want.decode(codes))
+    if extra > 0:
+        assert not torch.equal(got, dec.decode(codes))

@@ -253,13 +253,14 @@ __global__ __launch_bounds__(256) void codec_fragments_kernel(const uint8_t* __r
         make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
 }
 
-// codes -> bf16 [T, codebooks * dim]: codebook c's Q8_0 row of code [c, t] at columns c dim .. (an id outside the
+// codes -> bf16 [T, codebooks * dim]: codebook c's Q8_0 row of code [c, t] at columns c dim .. (an id outside that
 // table gives zeros), rounded to bf16 as the project_out product reads it.  One thread per 8 values.
 struct CdTables {
     const uint8_t* rows[32];
+    uint32_t count[32];  // rows of each table
 };
 __global__ __launch_bounds__(256) void codec_embed_kernel(const CdTables tables, const int64_t* __restrict__ codes,
-                                                          uint32_t books, uint32_t vocab, uint32_t dim, uint32_t len,
+                                                          uint32_t books, uint32_t dim, uint32_t len,
                                                           uint16_t* __restrict__ out) {
     const uint32_t per = dim / 8;
     const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(256) void codec_embed_kernel(const CdTables tables,
     const uint64_t t = idx / per / books;
     const int64_t id = codes[(uint64_t)c * len + t];
     uint4 o = make_uint4(0u, 0u, 0u, 0u);
-    if (id >= 0 && id < (int64_t)vocab) {
+    if (id >= 0 && id < (int64_t)tables.count[c]) {
         const uint8_t* p = tables.rows[c] + (size_t)id * ((dim + 31) / 32 * 34) + (size_t)(j / 4) * 34;
         const float d = f16_bits_to_f32(load_u16(p));
         const uint2 q = load_u2_ua(p + 2 + 8 * (j % 4));
@@ -319,9 +320,9 @@ static void cd_conv(const CdConvArgs& a, uint32_t taps, hipStream_t s) {
     else cd_dispatch<1, 32>(a, s);
 }
 
-// dims: codebooks, vocab, codebook_dim, latent, hidden, channels, blocks, then the blocks' strides
+// dims: codebooks, codebook_dim, latent, hidden, channels, blocks, then the blocks' strides
 struct CdDims {
-    uint32_t books, vocab, dim, latent, hidden, channels, blocks;
+    uint32_t books, dim, latent, hidden, channels, blocks;
     uint32_t strides[16];
     uint64_t len(uint32_t frames, uint32_t b) const {  // positions after b blocks
         uint64_t l = frames;
@@ -332,12 +333,11 @@ struct CdDims {
 
 static int cd_dims(const uint32_t* d, CdDims& o) {
     o.books = d[0];
-    o.vocab = d[1];
-    o.dim = d[2];
-    o.latent = d[3];
-    o.hidden = d[4];
-    o.channels = d[5];
-    o.blocks = d[6];
+    o.dim = d[1];
+    o.latent = d[2];
+    o.hidden = d[3];
+    o.channels = d[4];
+    o.blocks = d[5];
     if (o.books == 0 || o.books > 32 || o.blocks == 0 || o.blocks > 16) return T2H_ERR_UNSUPPORTED;
     if (o.dim == 0 || o.latent == 0 || o.hidden == 0 || o.channels == 0) return T2H_ERR_SHAPE;
     if (o.channels > (1u << 20) || o.latent > (1u << 20) || o.hidden > (1u << 20) || o.dim > (1u << 20))
@@ -346,7 +346,7 @@ static int cd_dims(const uint32_t* d, CdDims& o) {
         (o.channels >> o.blocks) == 0 || (o.channels & ((1u << o.blocks) - 1)))
         return T2H_ERR_UNSUPPORTED;
     for (uint32_t i = 0; i < o.blocks; ++i) {
-        o.strides[i] = d[7 + i];
+        o.strides[i] = d[6 + i];
         if (o.strides[i] < 2) return T2H_ERR_UNSUPPORTED;  // an output padding of stride % 2 needs stride > 1
         if (o.strides[i] > 1024) return T2H_ERR_UNSUPPORTED;
     }
@@ -405,10 +405,11 @@ extern "C" size_t t2h_codec_decode_workspace_bytes(const uint32_t* dims, uint32_
     return s.total;
 }
 
-extern "C" int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, uint32_t n_ptrs, const int64_t* codes,
-                                uint32_t frames, float eps, float* out, float* const* stages, void* workspace,
-                                size_t workspace_bytes, void* stream) {
-    if (!dims || !ptrs || !codes || !out || !workspace) return T2H_ERR_NULL;
+extern "C" int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, uint32_t n_ptrs,
+                                const uint32_t* table_rows, const int64_t* codes, uint32_t frames, float eps,
+                                float* out, float* const* stages, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+    if (!dims || !ptrs || !table_rows || !codes || !out || !workspace) return T2H_ERR_NULL;
     CdDims d;
     int st = cd_dims(dims, d);
     if (st) return st;
@@ -466,10 +467,13 @@ extern "C" int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, u
     };
 
     CdTables tables = {};
-    for (uint32_t c = 0; c < d.books; ++c) tables.rows[c] = reinterpret_cast<const uint8_t*>(*p++);
+    for (uint32_t c = 0; c < d.books; ++c) {
+        tables.rows[c] = reinterpret_cast<const uint8_t*>(*p++);
+        tables.count[c] = table_rows[c];
+    }
     const uint64_t work = (uint64_t)frames * d.books * (d.dim / 8);
     hipLaunchKernelGGL(codec_embed_kernel, dim3((uint32_t)((work + 255) / 256)), dim3(256), 0, s, tables, codes, d.books,
-                       d.vocab, d.dim, frames, gathered);
+                       d.dim, frames, gathered);
     T2H_LAUNCH_CHECK();
     const uint16_t* w = frag();
     conv(gathered, w, f32(), frames, d.books * d.dim, d.latent, 1, 0, nullptr, nullptr, latent, nullptr, nullptr);

@@ -116,8 +116,8 @@ class OmniVoiceAudioDecoder:
         self.device = torch.device(device)
         self.w = {n: (quantize_rows(a, self.device) if a.ndim == 2 else torch.from_numpy(a).to(self.device))
                   for n, a in dense.items()}
-        self._dims = (ctypes.c_uint32 * (7 + len(cfg.strides)))(cfg.codebooks, cfg.vocab, cfg.codebook_dim, cfg.latent,
-                                                                cfg.hidden, cfg.channels, len(cfg.strides), *cfg.strides)
+        self._dims = (ctypes.c_uint32 * (6 + len(cfg.strides)))(cfg.codebooks, cfg.codebook_dim, cfg.latent, cfg.hidden,
+                                                                cfg.channels, len(cfg.strides), *cfg.strides)
         fused = cfg.codebook_dim % 32 == 0 and cfg.latent % 64 == 0 and cfg.hidden % 64 == 0 and \
             self._workspace_bytes(1) > 0
         self._plan = self._lay_out() if fused else None
@@ -156,6 +156,7 @@ class OmniVoiceAudioDecoder:
         space = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         out = torch.empty(out_len(cfg, t), dtype=torch.float32, device=self.device)
         operands = (ctypes.c_void_p * len(self._plan))(*[x.data_ptr() for x in self._plan])
+        rows = (ctypes.c_uint32 * cfg.codebooks)(*[x.shape[0] for x in self._plan[:cfg.codebooks]])
         stage_ptrs = None
         if stages is not None:
             ch, length = cfg.channels, t
@@ -167,8 +168,9 @@ class OmniVoiceAudioDecoder:
             stages.extend(new)
             stage_arr = (ctypes.c_void_p * len(new))(*[x.data_ptr() for x in new])
             stage_ptrs = ctypes.addressof(stage_arr)
-        call("t2h_codec_decode", ctypes.addressof(self._dims), ctypes.addressof(operands), len(self._plan), ptr(codes), t, kernels.SNAKE_EPS,
-             ptr(out), stage_ptrs, ptr(space), nbytes, stream_handle())
+        call("t2h_codec_decode", ctypes.addressof(self._dims), ctypes.addressof(operands), len(self._plan),
+             ctypes.addressof(rows), ptr(codes), t, kernels.SNAKE_EPS, ptr(out), stage_ptrs, ptr(space), nbytes,
+             stream_handle())
         return out
 
     def _unit(self, x: torch.Tensor, p: str, dil: int) -> torch.Tensor:
