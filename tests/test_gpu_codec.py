@@ -127,3 +127,22 @@ def test_codec_tables_have_their_own_row_counts(device, extra):
     assert torch.equal(got, want.decode(codes))
     if extra > 0:
         assert not torch.equal(got, dec.decode(codes))
+
+
+# what the operators refuse of each kind of weight is refused by a decode that would run as one chain, too
+@pytest.mark.parametrize("name,change,error", [
+    ("b0.r0.a1", "half", TypeError), ("proj0.b", "double", TypeError), ("conv2.b", "half", TypeError),
+    ("b1.alpha", "longer", ValueError), ("b0.convt.b", "shorter", ValueError), ("fc2.b", "longer", ValueError),
+    ("cb1", "wider", ValueError), ("b0.r1.c1.w", "rows", ValueError), ("proj1.w", "wider", ValueError),
+    ("b1.convt.w", "rows", ValueError), ("conv2.w", "wider", ValueError)])
+def test_codec_refuses_weights_that_do_not_fit(device, name, change, error):
+    from torch2vk_amd.omnivoice.decoder import OmniVoiceAudioDecoder
+
+    _, cfg, dense, codes = _small_codec(device, 21)
+    a = dense[name]
+    a = {"half": lambda: a.astype(np.float16), "double": lambda: a.astype(np.float64),
+         "longer": lambda: np.concatenate([a, a]), "shorter": lambda: a[:a.shape[0] // 2].copy(),
+         "wider": lambda: np.concatenate([a] * 5, axis=1), "rows": lambda: np.concatenate([a, a])}[change]()
+    dec = OmniVoiceAudioDecoder(cfg, {**dense, name: a}, device)
+    with pytest.raises(error):
+        dec.decode(codes)

@@ -119,8 +119,25 @@ class OmniVoiceAudioDecoder:
         self._dims = (ctypes.c_uint32 * (6 + len(cfg.strides)))(cfg.codebooks, cfg.codebook_dim, cfg.latent, cfg.hidden,
                                                                 cfg.channels, len(cfg.strides), *cfg.strides)
         fused = cfg.codebook_dim % 32 == 0 and cfg.latent % 64 == 0 and cfg.hidden % 64 == 0 and \
-            self._workspace_bytes(1) > 0
+            self._workspace_bytes(1) > 0 and self._weights_fit()
         self._plan = self._lay_out() if fused else None
+
+    def _weights_fit(self) -> bool:
+        """Whether every weight is as t2h_codec_decode reads it through its pointer: Q8_0 rows of dense_shapes' sizes (a
+        codebook of any number of rows) and fp32 vectors.  Other weights run operator by operator, where each operator
+        takes or refuses them."""
+        for name, shape in dense_shapes(self.cfg).items():
+            t = self.w.get(name)
+            if not isinstance(t, torch.Tensor) or not t.is_cuda or not t.is_contiguous():
+                return False
+            if len(shape) == 1:
+                if t.dtype != torch.float32 or t.shape != shape or t.data_ptr() % 16:
+                    return False
+                continue
+            rows = t.shape[0] if name.startswith("cb") and t.dim() == 2 else shape[0]
+            if t.dtype != torch.uint8 or t.shape != (rows, -(-shape[1] // 32) * kernels.Q8_0_BYTES) or t.data_ptr() % 2:
+                return False
+        return True
 
     def _lay_out(self) -> list[torch.Tensor]:
         """t2h_codec_decode's operands in its order."""
