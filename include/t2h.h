@@ -457,29 +457,26 @@ int t2h_conv_transpose1d_q8_0(const float* x, const int64_t* x_strides, const vo
 
 /* The audio codec's whole decoder (run_audio_decode, src/models/quantized_omnivoice/dispatch/audio_decode.py:
  * 60-760) enqueued as one chain of fused launches: codes int64 [codebooks, frames] -> waveform fp32 [frames times the
- * strides' product].  dims: codebooks (<= 32), codebook_dim, latent, hidden, channels, blocks (<= 16), then each
- * block's stride (transposed conv of kernel 2 stride, padding ceil(stride / 2), output padding stride % 2);
- * every channel count % 8 == 0, channels halved by each block.  ptrs (codebooks + 9 + 21 blocks, in this order):
- * each codebook's Q8_0 table; project_out of all codebooks side by side (fragments, columns c dim + i), the sum of
- * its biases; fc2 (fragments), bias; conv1 (fragments, 7 taps), bias; block 0's alpha; per block: the transposed
- * conv's Q8_0 rows, its bias, unit 0's first alpha, and per unit: first conv (fragments, 7 taps), bias, second
- * alpha, second conv (fragments, 1 tap), bias, the alpha that follows (next unit, next block, or the last one);
- * then conv2 (fragments, 7 taps, one column), bias.  Fragments: bf16 [tap][step of 16 inputs][tile of 32
- * columns][64][8], lane l holding column l % 32 and inputs 8 (l / 32) .. + 7, inputs padded with zeros to 32 and
- * columns to 64.  table_rows: the rows of each codebook's table (a code outside its table embeds as zeros).
+ * strides' product].  dims: codebooks (<= 32), codebook_dim (% 32 == 0), latent, hidden, channels, blocks (<= 16), then
+ * each block's stride (transposed conv of kernel 2 stride, padding ceil(stride / 2), output padding stride % 2); every
+ * channel count % 8 == 0, channels halved by each block.
+ * A call enqueues parts part .. part + parts - 1 of 0: codes to conv1, 1 .. blocks: a block, blocks + 1: conv2; calls for
+ * one decode run in that order on one stream with the same arguments and workspace, so that a caller can look at the
+ * later parts' weights while the earlier ones run.
+ * ptrs (3 codebooks + 7 + 21 blocks, Q8_0 rows 2-byte and fp32 vectors 16-byte aligned), in this order: per codebook its
+ * table [table_rows[c], codebook_dim] (a code outside it embeds as zeros), project_out's rows and bias; fc2's rows and
+ * bias; conv1's rows [channels, 7 hidden] and bias; per block: the snake's alpha, the transposed conv's rows and bias, and
+ * per residual unit: first alpha, second alpha, first conv's rows (7 taps) and bias, second conv's rows (1 tap) and
+ * bias; then the last alpha, conv2's rows and bias.  A call reads its parts' pointers and the one that follows them (the
+ * next snake's alpha); the others may be NULL.
  * Rounding as in the operators one by one: convolution weights and inputs bf16, the rest fp32.
  * stages (or NULL): 1 + 4 blocks fp32 buffers for the activation after conv1, and after each block's transposed
  * conv and residual units.  workspace: t2h_codec_decode_workspace_bytes (0: dims or frames not supported), 256-byte
  * aligned. */
 size_t t2h_codec_decode_workspace_bytes(const uint32_t* dims, uint32_t frames);
-/* Q8_0 rows [n, cin taps] (element c taps + tap, rows of whole 34-byte blocks) as those fragments: bf16
- * [taps][ksteps][ceil(n / 64) 2][64][8], this matrix's inputs at steps kstep0 .. kstep0 + ceil(cin / 32) 2 - 1 (several
- * matrices side by side: cin % 32 == 0 for all but the last).  Each weight d q rounded once to bf16. */
-int t2h_conv_fragments_q8_0(const void* w, uint32_t n, uint32_t cin, uint32_t taps, uint32_t ksteps, uint32_t kstep0,
-                            void* out, void* stream);
-int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, uint32_t n_ptrs, const uint32_t* table_rows,
-                     const int64_t* codes, uint32_t frames, float eps, float* out, float* const* stages,
-                     void* workspace, size_t workspace_bytes, void* stream);
+int t2h_codec_decode(const uint32_t* dims, uint32_t part, uint32_t parts, const void* const* ptrs, uint32_t n_ptrs,
+                     const uint32_t* table_rows, const int64_t* codes, uint32_t frames, float eps, float* out,
+                     float* const* stages, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ----------------------------------------------- OmniVoice token loop --- */
 /* hidden fp32 [B, S, H] = sum over c < C of audio_w row (c * V + ids[b, c, s]) where audio_mask[b, s] != 0,

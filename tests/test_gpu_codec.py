@@ -146,3 +146,29 @@ def test_codec_refuses_weights_that_do_not_fit(device, name, change, error):
     dec = OmniVoiceAudioDecoder(cfg, {**dense, name: a}, device)
     with pytest.raises(error):
         dec.decode(codes)
+
+
+# 32 codebooks: more matrices than one layout launch takes; channels 48 and 24: steps and tiles that end inside
+@pytest.mark.parametrize("fields", [{}, {"codebooks": 32}, {"channels": 96, "hidden": 320}])
+def test_codec_decode_reads_the_weights_of_the_call(device, fields):
+    """Weights written in place or replaced between decodes are the ones that the next decode uses: the samples of a
+    decoder made with them."""
+    a, _, _, codes = _small_codec(device, 31, **fields)
+    b, _, _, _ = _small_codec(device, 32, **fields)
+    assert not torch.equal(a.decode(codes), b.decode(codes))
+    kept = {n: t.clone() for n, t in a.w.items()}
+    for i, (n, t) in enumerate(b.w.items()):
+        if i % 2:
+            a.w[n].copy_(t)
+        else:
+            a.w[n] = t.clone()
+    assert torch.equal(a.decode(codes), b.decode(codes))
+    for n in a.w:  # one at a time: each of them counts
+        before, a.w[n] = a.w[n], kept[n]
+        changed = a.decode(codes)
+        assert not torch.equal(changed, b.decode(codes)), n
+        a.w[n] = before
+    assert torch.equal(a.decode(codes), b.decode(codes))
+    a.w["b1.r2.a2"] = a.w["b1.r2.a2"].half()
+    with pytest.raises(TypeError):
+        a.decode(codes)

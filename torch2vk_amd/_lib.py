@@ -109,8 +109,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                          _vp]),
     "t2h_codec_decode_workspace_bytes": (_sz, [_vp, _u32]),
     "t2h_gemm_tiles": (_i32, [_i32, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _u32, _u32, _u32, _u32, _u32, _vp]),
-    "t2h_conv_fragments_q8_0": (_i32, [_vp, _u32, _u32, _u32, _u32, _u32, _vp, _vp]),
-    "t2h_codec_decode": (_i32, [_vp, _vp, _u32, _vp, _vp, _u32, _f32, _vp, _vp, _vp, _sz, _vp]),
+    "t2h_codec_decode": (_i32, [_vp, _u32, _u32, _vp, _u32, _vp, _vp, _u32, _f32, _vp, _vp, _vp, _sz, _vp]),
     "t2h_omnivoice_input_embed_q8_0": (_i32, [_vp, _u32, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _u32, _vp]),
     "t2h_omnivoice_cfg_score": (_i32, [_vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, _f32, _f32, _f32, _u32, _u32,
                                        ctypes.c_int64, _vp]),

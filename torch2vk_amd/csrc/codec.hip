@@ -12,13 +12,15 @@
 // convolution, which stays fp32) needs.  Rounding is where the operator-by-operator path has it: weights and
 // convolution inputs to bf16, everything else fp32.  Measured at 75 frames (1024 channels, strides 8, 5, 4, 2, 3):
 // 1806 us as about 200 launches of embedding, im2col, GEMM, snake and transposed convolution, bound by their
-// host work, by im2col's writes and by 256-wide GEMM tiles over 32 to 512 columns; 447 us as these 39, of
-// which the transposed convolutions take 161.
+// host work, by im2col's writes and by 256-wide GEMM tiles over 32 to 512 columns; 462 us as these 40 and two that
+// lay the weights out (8 + 5 us), of which the transposed convolutions take 160.
 //
-// Convolution weights are laid out once by the caller as bf16 fragments of v_mfma_f32_32x32x16_bf16,
-// [tap][channel step of 16][column tile of 32][lane][8]: lane l holds column l % 32, channels 8 (l / 32) + 0..7,
-// so a wave loads a fragment as one contiguous KB (channels padded with zeros to 32, columns to 64).
+// Convolution weights are read as bf16 fragments of v_mfma_f32_32x32x16_bf16, [tap][channel step of 16][column tile
+// of 32][lane][8]: lane l holds column l % 32, channels 8 (l / 32) + 0..7, so a wave loads a fragment as one contiguous
+// KB (channels padded with zeros to 32, columns to 64).  Each call lays them out from the packed rows into its workspace
+// (codec_layout_kernel), so a weight written between calls, by whatever means, is the one that the next call uses.
 #include "codec.h"
+#include "gemm_formats.h"
 
 namespace t2h {
 
@@ -227,44 +229,82 @@ __global__ __launch_bounds__(256) void codec_conv_kernel(const CdConvArgs a) {
     }
 }
 
-// Q8_0 rows [n, cin * taps] (element c taps + tap) -> fragments, channel steps kstep0 .. of `ksteps` per tap: thread
-// (tap, step, column tile, lane) converts its 8 weights, zero past the last channel and column.
-__global__ __launch_bounds__(256) void codec_fragments_kernel(const uint8_t* __restrict__ w, uint32_t n, uint32_t cin,
-                                                              uint32_t taps, uint32_t steps, uint32_t ntiles,
-                                                              uint32_t ksteps, uint32_t kstep0,
-                                                              uint16_t* __restrict__ out) {
-    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (uint64_t)taps * steps * ntiles * 64) return;
-    const uint32_t lane = (uint32_t)(idx % 64), tile = (uint32_t)(idx / 64 % ntiles);
-    const uint32_t step = (uint32_t)(idx / 64 / ntiles % steps), tap = (uint32_t)(idx / 64 / ntiles / steps);
-    const uint32_t col = tile * 32 + (lane & 31), c0 = step * 16 + 8 * (lane >> 5);
-    const uint8_t* row = w + (size_t)col * ((cin * taps + 31) / 32 * 34);
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        v[j] = 0.0f;
-        if (col < n && c0 + j < cin) {
-            const uint32_t e = (c0 + j) * taps + tap;
-            const uint8_t* b = row + (size_t)(e / 32) * 34;
-            v[j] = f16_bits_to_f32(load_u16(b)) * (float)(int8_t)b[2 + e % 32];
+// Weight rows -> fragments, all matrices of a call in one launch (Q8_0 rows [n, cin taps], element c taps + tap; several
+// matrices may lie side by side in one operand, each at its own channel steps).  A block converts 32 columns x 32
+// channels x 7 taps, or x 256 channels of one tap: 32 channels of a row are `taps` whole Q8_0 blocks, so a thread
+// converts one of a row's 7 or 8 consecutive blocks, every byte is read once, and the taps are picked apart in LDS.
+constexpr uint32_t CD_LAYOUTS = 32;  // matrices per launch
+struct CdLayout {
+    const uint8_t* w;
+    uint16_t* out;
+    uint32_t n, cin, taps;
+    uint32_t ksteps, kstep0;  // the operand's channel steps, and this matrix's first
+};
+struct CdLayouts {
+    CdLayout m[CD_LAYOUTS];
+    uint32_t first[64];  // first block of each matrix, then 2^32 - 1: one entry a lane
+};
+__host__ __device__ constexpr uint32_t cd_layout_groups(uint32_t taps) { return taps == 1 ? 8 : 1; }  // of 32 channels
+__global__ __launch_bounds__(256) void codec_layout_kernel(const CdLayouts a) {
+    constexpr uint32_t PITCH = 2 * 129;  // bf16 per LDS row of 8 blocks: the 32 rows of a read lie in distinct banks
+    __shared__ uint32_t ls[32 * PITCH / 2];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t i = __builtin_amdgcn_readfirstlane(__popcll(__ballot(a.first[lane] <= blockIdx.x)) - 1);
+    const uint32_t n = a.m[i].n, cin = a.m[i].cin, taps = a.m[i].taps, b = blockIdx.x - a.first[i];
+    const uint32_t ntiles = (n + 63) / 64 * 2, tile = b % ntiles, groups = cd_layout_groups(taps);
+    const uint32_t group0 = b / ntiles * groups, blocks = (cin * taps + 31) / 32;
+    {
+        const uint32_t row = tid / 8, k = tid % 8, col = tile * 32 + row, blk = group0 * taps + k;
+        GemmQ80::Raw r = {};
+        r.inside = col < n && k < groups * taps && blk < blocks;  // others: zeros
+        if (r.inside) {
+            const uint8_t* p = a.m[i].w + ((size_t)col * blocks + blk) * 34;
+            r.d = load_u16(p);
+            r.q0 = load_u4_ua(p + 2);
+            r.q1 = load_u4_ua(p + 18);
         }
+        uint32_t o[16];
+        GemmQ80::convert(r, 0, 0, o);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) ls[row * (PITCH / 2) + 16 * k + j] = o[j];
     }
-    *reinterpret_cast<uint4*>(out + ((((size_t)tap * ksteps + kstep0 + step) * ntiles + tile) * 64 + lane) * 8) =
-        make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+    __syncthreads();
+    const uint16_t* row = reinterpret_cast<const uint16_t*>(ls) + (lane & 31) * PITCH;
+    for (uint32_t u = wave; u < 2 * taps * groups; u += 4) {
+        const uint32_t step = u & 1, tap = taps == 1 ? 0 : u >> 1, local = taps == 1 ? u >> 1 : 0;
+        if (32 * (group0 + local) >= cin) break;  // past the last step
+        const uint32_t c = 32 * local + 16 * step + 8 * (lane >> 5);  // cin % 8 == 0: 8 channels are all inside or none
+        const uint32_t keep = 32 * group0 + c < cin ? 0xffffffffu : 0u;
+        uint32_t f[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            f[j] = ((uint32_t)row[(c + 2 * j) * taps + tap] | (uint32_t)row[(c + 2 * j + 1) * taps + tap] << 16) & keep;
+        const size_t at = ((size_t)tap * a.m[i].ksteps + a.m[i].kstep0 + 2 * (group0 + local) + step) * ntiles + tile;
+        *reinterpret_cast<uint4*>(a.m[i].out + (at * 64 + lane) * 8) = make_uint4(f[0], f[1], f[2], f[3]);
+    }
 }
 
 // codes -> bf16 [T, codebooks * dim]: codebook c's Q8_0 row of code [c, t] at columns c dim .. (an id outside that
-// table gives zeros), rounded to bf16 as the project_out product reads it.  One thread per 8 values.
+// table gives zeros), rounded to bf16 as the project_out product reads it.  One thread per 8 values; `latent` threads
+// more sum the codebooks' biases.
 struct CdTables {
     const uint8_t* rows[32];
     uint32_t count[32];  // rows of each table
+    const float* bias[32];
 };
 __global__ __launch_bounds__(256) void codec_embed_kernel(const CdTables tables, const int64_t* __restrict__ codes,
-                                                          uint32_t books, uint32_t dim, uint32_t len,
-                                                          uint16_t* __restrict__ out) {
+                                                          uint32_t books, uint32_t dim, uint32_t len, uint32_t latent,
+                                                          uint16_t* __restrict__ out, float* __restrict__ bias) {
     const uint32_t per = dim / 8;
-    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (uint64_t)len * books * per) return;
+    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x, gathers = (uint64_t)len * books * per;
+    if (idx >= gathers) {
+        const uint64_t i = idx - gathers;
+        if (i >= latent) return;
+        float v = tables.bias[0][i];
+        for (uint32_t c = 1; c < books; ++c) v += tables.bias[c][i];
+        bias[i] = v;
+        return;
+    }
     const uint32_t j = (uint32_t)(idx % per), c = (uint32_t)(idx / per % books);
     const uint64_t t = idx / per / books;
     const int64_t id = codes[(uint64_t)c * len + t];
@@ -342,7 +382,7 @@ static int cd_dims(const uint32_t* d, CdDims& o) {
     if (o.dim == 0 || o.latent == 0 || o.hidden == 0 || o.channels == 0) return T2H_ERR_SHAPE;
     if (o.channels > (1u << 20) || o.latent > (1u << 20) || o.hidden > (1u << 20) || o.dim > (1u << 20))
         return T2H_ERR_UNSUPPORTED;
-    if (o.dim % 8 || o.latent % 8 || o.hidden % 8 || (o.channels >> o.blocks) % 8 ||
+    if (o.dim % 32 || o.latent % 8 || o.hidden % 8 || (o.channels >> o.blocks) % 8 ||
         (o.channels >> o.blocks) == 0 || (o.channels & ((1u << o.blocks) - 1)))
         return T2H_ERR_UNSUPPORTED;
     for (uint32_t i = 0; i < o.blocks; ++i) {
@@ -353,10 +393,15 @@ static int cd_dims(const uint32_t* d, CdDims& o) {
     return T2H_OK;
 }
 
+// bf16 values of one operand's fragments
+static uint64_t cd_fragments(uint32_t cin, uint32_t n, uint32_t taps) {
+    return (uint64_t)taps * ((cin + 31) / 32 * 2) * ((n + 63) / 64 * 2) * 512;
+}
+
 // workspace: bf16 gathered rows, bf16 sums, bf16 hidden, then per position and channel of the widest point two
-// fp32 and two bf16 activations
+// fp32 and two bf16 activations, then the summed bias and the weights' fragments
 struct CdSpace {
-    uint64_t gather, latent, hidden, act, total;  // byte sizes; act: elements of the widest activation
+    uint64_t gather, latent, hidden, act, bias, total;  // byte sizes; act: elements of the widest activation
 };
 static int cd_space(const CdDims& d, uint32_t frames, CdSpace& s) {
     auto up = [](uint64_t v) { return (v + 255) / 256 * 256; };
@@ -373,30 +418,20 @@ static int cd_space(const CdDims& d, uint32_t frames, CdSpace& s) {
     }
     if (s.act > 0x7fffffffull || (uint64_t)frames * d.books * d.dim > 0x7fffffffull) return T2H_ERR_SHAPE;
     s.act = up(s.act);
-    s.total = s.gather + s.latent + s.hidden + s.act * (4 + 4 + 2 + 2);
+    s.bias = up(4ull * d.latent);
+    uint64_t frags = cd_fragments(d.books * d.dim, d.latent, 1) + cd_fragments(d.latent, d.hidden, 1) +
+                     cd_fragments(d.hidden, d.channels, CD_TAPS) + cd_fragments(d.channels >> d.blocks, 1, CD_TAPS);
+    for (uint32_t b = 1; b <= d.blocks; ++b)
+        frags += 3 * (cd_fragments(d.channels >> b, d.channels >> b, CD_TAPS) +
+                      cd_fragments(d.channels >> b, d.channels >> b, 1));
+    if (frags > 1ull << 40) return T2H_ERR_SHAPE;  // (a layout block converts 1024 or more: 2^30 blocks at most)
+    s.total = s.gather + s.latent + s.hidden + s.act * (4 + 4 + 2 + 2) + s.bias + 2 * frags;
     return T2H_OK;
 }
 
 }  // namespace t2h
 
 using namespace t2h;
-
-extern "C" int t2h_conv_fragments_q8_0(const void* w, uint32_t n, uint32_t cin, uint32_t taps, uint32_t ksteps,
-                                       uint32_t kstep0, void* out, void* stream) {
-    if (!w || !out) return T2H_ERR_NULL;
-    if (n == 0 || cin == 0 || taps == 0) return T2H_ERR_SHAPE;
-    if ((uint64_t)cin * taps > 0x7fffffffu || n > 0x7fffff00u) return T2H_ERR_SHAPE;
-    const uint32_t steps = (cin + 31) / 32 * 2, ntiles = (n + 63) / 64 * 2;
-    if (kstep0 > ksteps || steps > ksteps - kstep0) return T2H_ERR_ARG;
-    if (reinterpret_cast<uintptr_t>(w) % 2 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0) return T2H_ERR_ALIGN;
-    const uint64_t threads = (uint64_t)taps * steps * ntiles * 64;
-    if (threads / 256 >= 0x7fffffffu) return T2H_ERR_SHAPE;
-    hipLaunchKernelGGL(codec_fragments_kernel, dim3((uint32_t)((threads + 255) / 256)), dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint8_t*>(w), n, cin, taps, steps,
-                       ntiles, ksteps, kstep0, reinterpret_cast<uint16_t*>(out));
-    T2H_LAUNCH_CHECK();
-    return T2H_OK;
-}
 
 extern "C" size_t t2h_codec_decode_workspace_bytes(const uint32_t* dims, uint32_t frames) {
     CdDims d;
@@ -405,16 +440,21 @@ extern "C" size_t t2h_codec_decode_workspace_bytes(const uint32_t* dims, uint32_
     return s.total;
 }
 
-extern "C" int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, uint32_t n_ptrs,
-                                const uint32_t* table_rows, const int64_t* codes, uint32_t frames, float eps,
-                                float* out, float* const* stages, void* workspace, size_t workspace_bytes,
+extern "C" int t2h_codec_decode(const uint32_t* dims, uint32_t part, uint32_t parts, const void* const* ptrs,
+                                uint32_t n_ptrs, const uint32_t* table_rows, const int64_t* codes, uint32_t frames,
+                                float eps, float* out, float* const* stages, void* workspace, size_t workspace_bytes,
                                 void* stream) {
     if (!dims || !ptrs || !table_rows || !codes || !out || !workspace) return T2H_ERR_NULL;
     CdDims d;
     int st = cd_dims(dims, d);
     if (st) return st;
-    if (n_ptrs != d.books + 6 + d.blocks * 21 + 3) return T2H_ERR_ARG;
-    for (uint32_t i = 0; i < n_ptrs; ++i)
+    if (part >= d.blocks + 2 || parts == 0 || parts > d.blocks + 2 - part) return T2H_ERR_ARG;
+    const uint32_t end = part + parts;
+    // the operands of part q start at at(q); the first of a block and of the last part is the snake of the part before
+    auto at = [&](uint32_t q) { return q == 0 ? 0 : 3 * d.books + 4 + 21 * (q - 1); };
+    const uint32_t n_all = at(d.blocks + 1) + 3;
+    if (n_ptrs != n_all) return T2H_ERR_ARG;
+    for (uint32_t i = at(part); i < (end < d.blocks + 2 ? at(end) + 1 : n_all); ++i)
         if (!ptrs[i]) return T2H_ERR_NULL;
     if (frames == 0) return T2H_ERR_SHAPE;
     if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0) return T2H_ERR_ALIGN;
@@ -439,10 +479,49 @@ extern "C" int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, u
     float* xr = reinterpret_cast<float*>(take(4 * sp.act));   // residual stream of a block
     uint16_t* s1 = reinterpret_cast<uint16_t*>(take(2 * sp.act));
     uint16_t* s2 = reinterpret_cast<uint16_t*>(take(2 * sp.act));
+    float* bias0 = reinterpret_cast<float*>(take(sp.bias));
 
-    const void* const* p = ptrs;
-    auto f32 = [&]() { return reinterpret_cast<const float*>(*p++); };
-    auto frag = [&]() { return reinterpret_cast<const uint16_t*>(*p++); };
+    auto f32 = [&](uint32_t i) { return reinterpret_cast<const float*>(ptrs[i]); };
+    // the fragments of this call's parts, and the launches that lay them out
+    CdLayouts lay;
+    uint32_t lay_count = 0, lay_blocks = 0;
+    uint16_t* front[3] = {};
+    uint16_t* units[16][3][2] = {};
+    uint16_t* last = nullptr;
+    auto lay_flush = [&]() {
+        if (lay_count == 0) return;
+        for (uint32_t i = lay_count; i < 64; ++i) lay.first[i] = 0xffffffffu;
+        hipLaunchKernelGGL(codec_layout_kernel, dim3(lay_blocks), dim3(256), 0, s, lay);
+        lay_count = lay_blocks = 0;
+    };
+    auto lay_add = [&](uint32_t i, uint16_t* to, uint32_t cin, uint32_t n, uint32_t taps, uint32_t ksteps, uint32_t kstep0) {
+        if (lay_count == CD_LAYOUTS) lay_flush();
+        lay.m[lay_count] = {reinterpret_cast<const uint8_t*>(ptrs[i]), to, n, cin, taps, ksteps, kstep0};
+        lay.first[lay_count++] = lay_blocks;
+        lay_blocks += (n + 63) / 64 * 2 * ((cin + 32 * cd_layout_groups(taps) - 1) / (32 * cd_layout_groups(taps)));
+    };
+    auto lay_one = [&](uint32_t q, uint32_t i, uint32_t cin, uint32_t n, uint32_t taps) {
+        uint16_t* to = reinterpret_cast<uint16_t*>(take(2 * cd_fragments(cin, n, taps)));
+        if (q >= part && q < end) lay_add(i, to, cin, n, taps, (cin + 31) / 32 * 2, 0);
+        return to;
+    };
+    const uint32_t dsteps = d.dim / 32 * 2;
+    front[0] = reinterpret_cast<uint16_t*>(take(2 * cd_fragments(d.books * d.dim, d.latent, 1)));
+    if (part == 0)
+        for (uint32_t c = 0; c < d.books; ++c)
+            lay_add(3 * c + 1, front[0], d.dim, d.latent, 1, d.books * dsteps, c * dsteps);
+    front[1] = lay_one(0, 3 * d.books, d.latent, d.hidden, 1);
+    front[2] = lay_one(0, 3 * d.books + 2, d.hidden, d.channels, CD_TAPS);
+    for (uint32_t b = 0; b < d.blocks; ++b)
+        for (uint32_t u = 0; u < 3; ++u) {
+            const uint32_t i = at(b + 1) + 3 + 6 * u, co = d.channels >> (b + 1);
+            units[b][u][0] = lay_one(b + 1, i + 2, co, co, CD_TAPS);
+            units[b][u][1] = lay_one(b + 1, i + 4, co, co, 1);
+        }
+    last = lay_one(d.blocks + 1, at(d.blocks + 1) + 1, d.channels >> d.blocks, 1, CD_TAPS);
+    lay_flush();
+    T2H_LAUNCH_CHECK();
+
     // one convolution: alpha null leaves the result as it is
     auto conv = [&](const uint16_t* x, const uint16_t* w, const float* bias, uint64_t len, uint32_t cin, uint32_t n,
                     uint32_t taps, uint32_t dil, const float* res, float* raw, uint16_t* bf, float* snaked,
@@ -466,57 +545,50 @@ extern "C" int t2h_codec_decode(const uint32_t* dims, const void* const* ptrs, u
         cd_conv(a, taps, s);
     };
 
-    CdTables tables = {};
-    for (uint32_t c = 0; c < d.books; ++c) {
-        tables.rows[c] = reinterpret_cast<const uint8_t*>(*p++);
-        tables.count[c] = table_rows[c];
+    if (part == 0) {
+        CdTables tables = {};
+        for (uint32_t c = 0; c < d.books; ++c) {
+            tables.rows[c] = reinterpret_cast<const uint8_t*>(ptrs[3 * c]);
+            tables.count[c] = table_rows[c];
+            tables.bias[c] = f32(3 * c + 2);
+        }
+        const uint64_t work = (uint64_t)frames * d.books * (d.dim / 8) + d.latent;
+        hipLaunchKernelGGL(codec_embed_kernel, dim3((uint32_t)((work + 255) / 256)), dim3(256), 0, s, tables, codes,
+                           d.books, d.dim, frames, d.latent, gathered, bias0);
+        T2H_LAUNCH_CHECK();
+        const uint32_t i = 3 * d.books;
+        conv(gathered, front[0], bias0, frames, d.books * d.dim, d.latent, 1, 0, nullptr, nullptr, latent, nullptr, nullptr);
+        conv(latent, front[1], f32(i + 1), frames, d.latent, d.hidden, 1, 0, nullptr, nullptr, hidden, nullptr, nullptr);
+        conv(hidden, front[2], f32(i + 3), frames, d.hidden, d.channels, CD_TAPS, 1, nullptr,
+             stages ? stages[0] : nullptr, nullptr, xs, f32(i + 4));
+        T2H_LAUNCH_CHECK();
     }
-    const uint64_t work = (uint64_t)frames * d.books * (d.dim / 8);
-    hipLaunchKernelGGL(codec_embed_kernel, dim3((uint32_t)((work + 255) / 256)), dim3(256), 0, s, tables, codes, d.books,
-                       d.dim, frames, gathered);
-    T2H_LAUNCH_CHECK();
-    const uint16_t* w = frag();
-    conv(gathered, w, f32(), frames, d.books * d.dim, d.latent, 1, 0, nullptr, nullptr, latent, nullptr, nullptr);
-    w = frag();
-    conv(latent, w, f32(), frames, d.latent, d.hidden, 1, 0, nullptr, nullptr, hidden, nullptr, nullptr);
-    w = frag();
-    const float* b1 = f32();
-    const float* alpha = f32();  // block 0's
-    conv(hidden, w, b1, frames, d.hidden, d.channels, CD_TAPS, 1, nullptr, stages ? stages[0] : nullptr, nullptr, xs,
-         alpha);
-    T2H_LAUNCH_CHECK();
-    uint64_t len = frames;
     static const uint32_t dils[3] = {1, 3, 9};
-    for (uint32_t b = 0; b < d.blocks; ++b) {
-        const uint32_t ch = d.channels >> b, co = ch / 2, stride = d.strides[b];
-        const void* wt = *p++;
-        const float* bt = f32();
+    for (uint32_t b = part == 0 ? 0 : part - 1; b < d.blocks && b + 1 < end; ++b) {
+        const uint32_t ch = d.channels >> b, co = ch / 2, stride = d.strides[b], first = at(b + 1);
+        const uint64_t li = d.len(frames, b), len = li * stride;
         float* x = stages ? stages[1 + 4 * b] : xr;
-        const int64_t strides[3] = {(int64_t)(len * ch), 1, (int64_t)ch};
-        const uint64_t lo = len * stride;
-        const float* a1 = f32();
-        st = conv_transpose1d_q8_0_launch(xs, strides, wt, bt, x, 1, ch, (uint32_t)len, co, 2 * stride, stride,
-                                          (stride + 1) / 2, (uint32_t)lo, s1, a1, eps, stream);
+        const int64_t strides[3] = {(int64_t)(li * ch), 1, (int64_t)ch};
+        st = conv_transpose1d_q8_0_launch(xs, strides, ptrs[first + 1], f32(first + 2), x, 1, ch, (uint32_t)li, co,
+                                          2 * stride, stride, (stride + 1) / 2, (uint32_t)len, s1, f32(first + 3), eps,
+                                          stream);
         if (st) return st;
-        len = lo;
         for (uint32_t u = 0; u < 3; ++u) {
-            const uint16_t* w1 = frag();
-            const float* bias1 = f32();
-            const float* a2 = f32();
-            const uint16_t* w2 = frag();
-            const float* bias2 = f32();
-            const float* next = f32();  // the next unit's, the next block's, or the final alpha
-            conv(s1, w1, bias1, len, co, co, CD_TAPS, dils[u], nullptr, nullptr, s2, nullptr, a2);
-            const bool last = u == 2, end = last && b + 1 == d.blocks;
-            float* raw = stages ? stages[2 + 4 * b + u] : (last ? nullptr : xr);
-            conv(s2, w2, bias2, len, co, co, 1, 0, x, raw, last && !end ? nullptr : s1, last && !end ? xs : nullptr,
-                 next);
+            const uint32_t i = first + 3 + 6 * u;  // a1, a2, c1, its bias, c2, its bias; then the next snake's alpha
+            conv(s1, units[b][u][0], f32(i + 3), len, co, co, CD_TAPS, dils[u], nullptr, nullptr, s2, nullptr, f32(i + 1));
+            const bool third = u == 2, final = third && b + 1 == d.blocks;
+            float* raw = stages ? stages[2 + 4 * b + u] : (third ? nullptr : xr);
+            conv(s2, units[b][u][1], f32(i + 5), len, co, co, 1, 0, x, raw, third && !final ? nullptr : s1,
+                 third && !final ? xs : nullptr, f32(i + 6));
             x = raw;
             T2H_LAUNCH_CHECK();
         }
     }
-    w = frag();
-    conv(s1, w, f32(), len, d.channels >> d.blocks, 1, CD_TAPS, 1, nullptr, out, nullptr, nullptr, nullptr);
-    T2H_LAUNCH_CHECK();
+    if (end == d.blocks + 2) {
+        const uint32_t i = at(d.blocks + 1);
+        conv(s1, last, f32(i + 2), d.len(frames, d.blocks), d.channels >> d.blocks, 1, CD_TAPS, 1, nullptr, out, nullptr,
+             nullptr, nullptr);
+        T2H_LAUNCH_CHECK();
+    }
     return T2H_OK;
 }

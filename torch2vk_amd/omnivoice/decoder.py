@@ -18,6 +18,7 @@ from __future__ import annotations
 import ctypes
 import math
 from dataclasses import dataclass
+from operator import attrgetter, itemgetter
 
 import numpy as np
 import torch
@@ -96,85 +97,85 @@ def quantize_rows(w: np.ndarray, device) -> torch.Tensor:
     return kernels.quantize(torch.from_numpy(full).to(device), "q8_0")
 
 
-def conv_fragments(rows: list[torch.Tensor], cin: int, taps: int) -> torch.Tensor:
-    """Q8_0 conv rows [n, cin * taps] (element c * taps + k), several matrices' inputs side by side, as the bf16
-    fragments t2h_codec_decode reads: [tap][step of 16 inputs][tile of 32 columns][64][8]."""
-    n, steps = int(rows[0].shape[0]), -(-cin // 32) * 2
-    out = torch.empty(taps, steps * len(rows), -(-n // 64) * 2, 64, 8, dtype=torch.bfloat16, device=rows[0].device)
-    for i, r in enumerate(rows):
-        call("t2h_conv_fragments_q8_0", ptr(r), n, cin, taps, steps * len(rows), steps * i, ptr(out), stream_handle())
-    return out
+_dtype, _is_cuda, _size = attrgetter("dtype"), attrgetter("is_cuda"), torch.Tensor.size
+
+
+class _Operands:
+    """What t2h_codec_decode reads through its pointers for parts ``part`` .. ``part + parts - 1`` of a decode: the names
+    of dense_shapes from index ``first``, their dtypes and their packed sizes."""
+
+    def __init__(self, cfg: AudioDecoderConfig, part: int, parts: int) -> None:
+        def at(q: int) -> int:  # where part q's operands start; a part also reads the alpha that follows it
+            return 0 if q == 0 else 3 * cfg.codebooks + 4 + 21 * (q - 1)
+
+        every = list(dense_shapes(cfg).items())
+        self.part, self.parts, self.first = part, parts, at(part)
+        shapes = every[self.first:at(part + parts) + 1 if part + parts < len(cfg.strides) + 2 else len(every)]
+        self.last = self.first + len(shapes)
+        self.tensors = itemgetter(*(name for name, _ in shapes))
+        self.dtypes = [torch.float32 if len(s) == 1 else torch.uint8 for _, s in shapes]
+        self.sizes = [s if len(s) == 1 else (s[0], -(-s[1] // 32) * kernels.Q8_0_BYTES) for _, s in shapes]
+        self.tables = [i for i, (name, _) in enumerate(shapes) if name.startswith("cb")]  # of any number of rows
+        self.vectors = [i for i, (_, s) in enumerate(shapes) if len(s) == 1]
+
+    def pointers(self, w: dict[str, torch.Tensor]) -> tuple[list[int], list[int]] | None:
+        """(pointers, rows of the codebooks), or None where a weight is not as the chain reads it.  Looked at on every
+        call (about 0.4 us a weight): entries of ``w`` can be replaced, resized or cast at any time."""
+        try:
+            ts = self.tensors(w)
+        except KeyError:
+            return None
+        if not all(issubclass(t, torch.Tensor) for t in set(map(type, ts))) or list(map(_dtype, ts)) != self.dtypes:
+            return None
+        sizes = list(map(_size, ts))
+        rows = []
+        for i in self.tables:
+            if len(sizes[i]) != 2:
+                return None
+            rows.append(sizes[i][0])
+            sizes[i] = (self.sizes[i][0], sizes[i][1])
+        if sizes != self.sizes or not all(map(_is_cuda, ts)) or not all(map(torch.Tensor.is_contiguous, ts)):
+            return None
+        ptrs = list(map(torch.Tensor.data_ptr, ts))
+        if any(p & 1 for p in ptrs) or any(ptrs[i] & 15 for i in self.vectors) or 0 in ptrs:
+            return None
+        return ptrs, rows
 
 
 class OmniVoiceAudioDecoder:
-    """``w`` holds the packed weights.  The convolutions are also laid out as bf16 fragments when the decoder is
-    made (t2h_codec_decode then runs a whole decode as about 40 launches); channel counts that path is not built
-    for run operator by operator."""
+    """``w`` holds the packed weights; a decode reads them as they are when it is called.  Where they have the configured
+    shapes it is one chain of about 40 launches (t2h_codec_decode); other shapes, and channel counts that chain is not
+    built for, run operator by operator."""
 
     def __init__(self, cfg: AudioDecoderConfig, dense: dict[str, np.ndarray], device) -> None:
         self.cfg = cfg
         self.device = torch.device(device)
         self.w = {n: (quantize_rows(a, self.device) if a.ndim == 2 else torch.from_numpy(a).to(self.device))
                   for n, a in dense.items()}
-        self._dims = (ctypes.c_uint32 * (6 + len(cfg.strides)))(cfg.codebooks, cfg.codebook_dim, cfg.latent, cfg.hidden,
-                                                                cfg.channels, len(cfg.strides), *cfg.strides)
+        blocks = len(cfg.strides)
+        self._dims = (ctypes.c_uint32 * (6 + blocks))(cfg.codebooks, cfg.codebook_dim, cfg.latent, cfg.hidden,
+                                                      cfg.channels, blocks, *cfg.strides)
         fused = cfg.codebook_dim % 32 == 0 and cfg.latent % 64 == 0 and cfg.hidden % 64 == 0 and \
-            self._workspace_bytes(1) > 0 and self._weights_fit()
-        self._plan = self._lay_out() if fused else None
-
-    def _weights_fit(self) -> bool:
-        """Whether every weight is as t2h_codec_decode reads it through its pointer: Q8_0 rows of dense_shapes' sizes (a
-        codebook of any number of rows) and fp32 vectors.  Other weights run operator by operator, where each operator
-        takes or refuses them."""
-        for name, shape in dense_shapes(self.cfg).items():
-            t = self.w.get(name)
-            if not isinstance(t, torch.Tensor) or not t.is_cuda or not t.is_contiguous():
-                return False
-            if len(shape) == 1:
-                if t.dtype != torch.float32 or t.shape != shape or t.data_ptr() % 16:
-                    return False
-                continue
-            rows = t.shape[0] if name.startswith("cb") and t.dim() == 2 else shape[0]
-            if t.dtype != torch.uint8 or t.shape != (rows, -(-shape[1] // 32) * kernels.Q8_0_BYTES) or t.data_ptr() % 2:
-                return False
-        return True
-
-    def _lay_out(self) -> list[torch.Tensor]:
-        """t2h_codec_decode's operands in its order."""
-        cfg, w = self.cfg, self.w
-        bias = w["proj0.b"]
-        for c in range(1, cfg.codebooks):
-            bias = bias + w[f"proj{c}.b"]
-        plan = [w[f"cb{c}"] for c in range(cfg.codebooks)]
-        plan += [conv_fragments([w[f"proj{c}.w"] for c in range(cfg.codebooks)], cfg.codebook_dim, 1), bias]
-        plan += [conv_fragments([w["fc2.w"]], cfg.latent, 1), w["fc2.b"]]
-        plan += [conv_fragments([w["conv1.w"]], cfg.hidden, 7), w["conv1.b"], w["b0.alpha"]]
-        ch, blocks, units = cfg.channels, len(cfg.strides), len(DILATIONS)
-        for i in range(blocks):
-            ch //= 2
-            plan += [w[f"b{i}.convt.w"], w[f"b{i}.convt.b"], w[f"b{i}.r0.a1"]]
-            for j in range(units):
-                p = f"b{i}.r{j}."
-                if j + 1 < units:
-                    after = f"b{i}.r{j + 1}.a1"
-                else:
-                    after = f"b{i + 1}.alpha" if i + 1 < blocks else "final.alpha"
-                plan += [conv_fragments([w[p + "c1.w"]], ch, 7), w[p + "c1.b"], w[p + "a2"],
-                         conv_fragments([w[p + "c2.w"]], ch, 1), w[p + "c2.b"], w[after]]
-        return plan + [conv_fragments([w["conv2.w"]], ch, 7), w["conv2.b"]]
+            self._workspace_bytes(1) > 0
+        # in two calls: the host looks at the later blocks' weights while the GPU runs the first part
+        self._plan = [_Operands(cfg, 0, 2), _Operands(cfg, 2, blocks)] if fused else None
 
     def _workspace_bytes(self, frames: int) -> int:
         """Bytes t2h_codec_decode needs (0: more frames than it takes)."""
         return int(_lib.lib().t2h_codec_decode_workspace_bytes(ctypes.addressof(self._dims), frames))
 
-    def _decode_fused(self, codes: torch.Tensor, nbytes: int, stages: list | None) -> torch.Tensor:
+    def _decode_fused(self, codes: torch.Tensor, nbytes: int, stages: list | None) -> torch.Tensor | None:
+        """The decode as t2h_codec_decode's chain, or None where a weight does not fit it."""
         cfg, t = self.cfg, int(codes.shape[1])
+        found = self._plan[0].pointers(self.w)
+        if found is None:
+            return None
+        n = self._plan[-1].last
+        operands, rows = (ctypes.c_void_p * n)(), (ctypes.c_uint32 * cfg.codebooks)(*found[1])
         codes = codes[:cfg.codebooks].contiguous()
         space = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         out = torch.empty(out_len(cfg, t), dtype=torch.float32, device=self.device)
-        operands = (ctypes.c_void_p * len(self._plan))(*[x.data_ptr() for x in self._plan])
-        rows = (ctypes.c_uint32 * cfg.codebooks)(*[x.shape[0] for x in self._plan[:cfg.codebooks]])
-        stage_ptrs = None
+        new, stage_ptrs = [], None
         if stages is not None:
             ch, length = cfg.channels, t
             new = [torch.empty(1, t, ch, dtype=torch.float32, device=self.device)]
@@ -182,12 +183,19 @@ class OmniVoiceAudioDecoder:
                 ch, length = ch // 2, length * s
                 new += [torch.empty(1, length, ch, dtype=torch.float32, device=self.device)
                         for _ in range(1 + len(DILATIONS))]
-            stages.extend(new)
             stage_arr = (ctypes.c_void_p * len(new))(*[x.data_ptr() for x in new])
             stage_ptrs = ctypes.addressof(stage_arr)
-        call("t2h_codec_decode", ctypes.addressof(self._dims), ctypes.addressof(operands), len(self._plan),
-             ctypes.addressof(rows), ptr(codes), t, kernels.SNAKE_EPS, ptr(out), stage_ptrs, ptr(space), nbytes,
-             stream_handle())
+        for group in self._plan:
+            found = found or group.pointers(self.w)
+            if found is None:
+                return None  # what is enqueued writes only this call's own buffers
+            operands[group.first:group.last] = found[0]
+            found = None
+            call("t2h_codec_decode", ctypes.addressof(self._dims), group.part, group.parts, ctypes.addressof(operands), n,
+                 ctypes.addressof(rows), ptr(codes), t, kernels.SNAKE_EPS, ptr(out), stage_ptrs, ptr(space), nbytes,
+                 stream_handle())
+        if stages is not None:
+            stages.extend(new)
         return out
 
     def _unit(self, x: torch.Tensor, p: str, dil: int) -> torch.Tensor:
@@ -206,8 +214,9 @@ class OmniVoiceAudioDecoder:
         t = int(codes.shape[1])
         if self._plan is not None and 0 < t < 1 << 31 and codes.dim() == 2 and codes.shape[0] >= cfg.codebooks:
             nbytes = self._workspace_bytes(t)
-            if nbytes:
-                return self._decode_fused(codes, nbytes, stages)
+            out = self._decode_fused(codes, nbytes, stages) if nbytes else None
+            if out is not None:
+                return out
         acc = torch.zeros(t, cfg.latent, dtype=torch.float32, device=self.device)
         for c in range(cfg.codebooks):
             e = kernels.embedding_q8_0(w[f"cb{c}"], codes[c].contiguous(), cfg.codebook_dim)
