@@ -505,14 +505,18 @@ int t2h_omnivoice_token_update_topk(const int64_t* cand_tokens, const float* can
 /* conv2d without a patch matrix: out [batch, oh, ow, n] bf16 = act(conv(x, w) + bias), act 0 or 1 (GELU), bias fp32
  * [n] or NULL, the same stride and zero padding on both axes.
  * t2h_conv2d_bf16: x [batch, h, w, channels] bf16, w_rows bf16 [n, kp], element (ky kw + kx) channels + c, kp =
- * kh kw channels rounded up to 64 and zeros past it; channels % 8 == 0, 64 <= channels < 65536, kh kw <= 24, kw <= w, a patch's kh rows of x under 2 GiB.  tile: -1 for the launch's own choice, 0 .. 3 for 64 x 64, 128 x 128 in three
- * and in two stages, 256 x 256.
+ * kh kw channels rounded up to 64 and zeros past it; channels % 8 == 0, 64 <= channels < 65536, kh kw <= 24, kw <= w, a
+ * patch's kh rows of x under 2 GiB.  tile: -1 for the launch's own choice, 0 .. 3 for 64 x 64, 128 x 128 in three and in
+ * two stages, 256 x 256.
+ * t2h_conv2d_rows_q8_0: those rows from w, Q8_0 rows [n, channels taps] (element channel taps + ky kw + kx), taps = kh kw
+ * <= 24; each weight d q rounded once to bf16.
  * t2h_conv2d_1ch_q8_0: x [batch, h, w] fp32 (rounded to bf16), w Q8_0 rows [n, 34] (kh kw <= 16 taps, then values that
  * are not read); n % 8 == 0.
  * Pointers 16-byte aligned (bias 4, Q8_0 rows 2, fp32 x 4); other shapes: T2H_ERR_UNSUPPORTED. */
 int t2h_conv2d_bf16(const void* x, const void* w_rows, const void* bias, int act, void* out, uint32_t batch, uint32_t h,
                     uint32_t w, uint32_t channels, uint32_t n, uint32_t kh, uint32_t kw, uint32_t stride, uint32_t pad,
                     int tile, void* stream);
+int t2h_conv2d_rows_q8_0(const void* w, uint32_t n, uint32_t channels, uint32_t taps, void* out, void* stream);
 int t2h_conv2d_1ch_q8_0(const void* x, const void* w, const void* bias, int act, void* out, uint32_t batch, uint32_t h,
                         uint32_t w_in, uint32_t n, uint32_t kh, uint32_t kw, uint32_t stride, uint32_t pad, void* stream);
 /* out = (x - mean) / sqrt(var + eps) * w + b per row (biased variance, two passes); x, out fp32 or bf16,

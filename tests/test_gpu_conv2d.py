@@ -76,3 +76,40 @@ def test_conv2d_1ch_matches_reference(shape, kernel, stride, pad, n):
     out = kernels.conv2d_1ch(x.cuda(), packed, bias.cuda(), kernel, stride, pad, act="gelu")
     w = _weights(packed, taps).view(n, 1, *kernel)
     _check(out, x.to(torch.bfloat16).double(), w, bias.double(), stride, pad, "gelu")
+
+
+# a whole stage of K and one that ends inside it; channels past one block's 512; channel counts off 8 and 32
+@pytest.mark.parametrize("n,c,taps", [(3, 64, 9), (5, 480, 9), (2, 1096, 24), (4, 36, 6), (3, 517, 3), (1, 8, 1)])
+def test_conv2d_rows_are_the_weights_tap_major(n, c, taps):
+    packed = _rows(torch.Generator().manual_seed(n + c), n, c * taps)
+    rows = kernels.conv2d_rows(packed, c, (1, taps)).cpu()
+    want = _weights(packed, c * taps).view(n, c, taps).transpose(1, 2).reshape(n, -1)
+    assert rows.shape == (n, -(-c * taps // 64) * 64)
+    assert torch.equal(rows[:, :c * taps].double(), want) and not rows[:, c * taps:].any()
+
+
+def test_encoder_front_end_reads_the_weights_of_the_call():
+    """Convolution weights written in place or replaced after an encoder was made are the ones that it uses."""
+    from torch2vk_amd.qwen3_asr.config import AudioEncoderConfig
+    from torch2vk_amd.qwen3_asr.encoder import Qwen3AudioEncoder, quantize_audio_weights, synthetic_audio_dense
+
+    cfg = AudioEncoderConfig(d_model=128, layers=1, heads=2, ffn=256, output_dim=128, conv_channels=64)
+    a, b = (Qwen3AudioEncoder(quantize_audio_weights(synthetic_audio_dense(cfg, seed=s), cfg, torch.device("cuda")))
+            for s in (1, 2))
+    g = torch.Generator().manual_seed(3)
+    mel = torch.randn(2, 1, cfg.mel_bins, 100, generator=g).cuda()
+    tokens = 100
+    for _ in range(3):
+        tokens = (tokens - 1) // 2 + 1
+    pos = torch.randn(2, tokens, cfg.d_model, generator=g).cuda()
+    want = b.frontend(mel, pos)
+    assert not torch.equal(a.frontend(mel, pos), want)
+    for name, t in b.weights.packed.items():
+        if "conv" in name and name.endswith("2.weight"):
+            a.weights.packed[name].copy_(t)
+        elif "conv" in name:
+            a.weights.packed[name] = t.clone()
+    for name, t in b.weights.vectors.items():
+        if "conv" in name:
+            a.weights.vectors[name].copy_(t)
+    assert torch.equal(a.frontend(mel, pos), want)

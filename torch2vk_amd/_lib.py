@@ -89,6 +89,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "t2h_im2col": (_i32, [_vp, _i32, _vp, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32,
                           _vp, _u32, _vp]),
     "t2h_conv2d_bf16": (_i32, [_vp, _vp, _vp, _i32, _vp] + [_u32] * 9 + [_i32, _vp]),
+    "t2h_conv2d_rows_q8_0": (_i32, [_vp, _u32, _u32, _u32, _vp, _vp]),
     "t2h_conv2d_1ch_q8_0": (_i32, [_vp, _vp, _vp, _i32, _vp] + [_u32] * 8 + [_vp]),
     "t2h_layer_norm": (_i32, [_vp, _i32, _vp, _vp, _vp, _i32, _u32, _u32, _f32, _vp]),
     "t2h_gelu": (_i32, [_vp, _i32, _vp, _i32, _u64, _vp]),

@@ -240,6 +240,50 @@ __global__ __launch_bounds__(CV_THREADS) void conv2d_kernel(const Conv2dArgs a) 
     }
 }
 
+// Q8_0 rows [n, c taps] (element c taps + tap) -> the weight rows above.  A block converts up to 512 channels of a row:
+// 32 channels are `taps` whole Q8_0 blocks, one a thread, and the taps are picked apart in LDS.  Laid out before every
+// convolution, so that it uses the weights as they are then: 480 rows of C 480, 9 taps, in 5 us.
+constexpr uint32_t CR_CHANNELS = 512, CR_MAX_TAPS = 24;
+__global__ __launch_bounds__(256) void conv2d_rows_kernel(const uint8_t* __restrict__ w, uint32_t c, uint32_t taps,
+                                                          uint32_t kp, uint16_t* __restrict__ out) {
+    __shared__ __align__(16) uint16_t ls[CR_CHANNELS * CR_MAX_TAPS];
+    const uint32_t c0 = blockIdx.y * CR_CHANNELS, cn = min(CR_CHANNELS, c - c0);
+    const uint32_t blocks = (c * taps + 31) / 32, b0 = c0 / 32 * taps, bn = min(CR_CHANNELS / 32 * taps, blocks - b0);
+    const uint8_t* src = w + ((size_t)blockIdx.x * blocks + b0) * 34;
+    for (uint32_t i = threadIdx.x; i < bn; i += 256) {
+        GemmQ80::Raw r;
+        r.d = load_u16(src + 34 * i);
+        r.inside = true;
+        r.q0 = load_u4_ua(src + 34 * i + 2);
+        r.q1 = load_u4_ua(src + 34 * i + 18);
+        uint32_t o[16];
+        GemmQ80::convert(r, 0, 0, o);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            *reinterpret_cast<uint4*>(ls + 32 * i + 8 * j) = make_uint4(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
+    }
+    __syncthreads();
+    uint16_t* row = out + (size_t)blockIdx.x * kp;
+    const uint32_t chunks = (cn + 7) / 8;
+    for (uint32_t i = threadIdx.x; i < chunks * taps; i += 256) {
+        const uint32_t tap = i / chunks, ch = i % chunks * 8;
+        uint16_t v[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) v[j] = ls[min(ch + j, cn - 1) * taps + tap];
+        uint16_t* dst = row + (size_t)tap * c + c0 + ch;
+        if (c % 8 == 0) {
+            *reinterpret_cast<uint4*>(dst) =
+                make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16,
+                           v[6] | (uint32_t)v[7] << 16);
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j)
+                if (ch + j < cn) dst[j] = v[j];
+        }
+    }
+    if (blockIdx.y == 0 && c * taps + threadIdx.x < kp) row[c * taps + threadIdx.x] = 0;  // fewer than 64
+}
+
 // --------------------------------------------------------- one channel ----
 
 struct Conv2d1Args {
@@ -402,6 +446,18 @@ extern "C" int t2h_conv2d_bf16(const void* x, const void* w_rows, const void* bi
     else if (tile == 2) conv2d_launch<2, 2, 2>(a, s);
     else if (tile == 3) conv2d_launch<4, 4, 2>(a, s);
     else return T2H_ERR_UNSUPPORTED;
+    T2H_LAUNCH_CHECK();
+    return T2H_OK;
+}
+
+extern "C" int t2h_conv2d_rows_q8_0(const void* w, uint32_t n, uint32_t channels, uint32_t taps, void* out, void* stream) {
+    if (!w || !out) return T2H_ERR_NULL;
+    if (n == 0 || channels == 0 || taps == 0) return T2H_ERR_SHAPE;
+    if (taps > CR_MAX_TAPS || channels > 0xffff || n > 0x7fffffffu) return T2H_ERR_UNSUPPORTED;
+    if ((reinterpret_cast<uintptr_t>(w) & 1) != 0 || (reinterpret_cast<uintptr_t>(out) & 15) != 0) return T2H_ERR_ALIGN;
+    hipLaunchKernelGGL(conv2d_rows_kernel, dim3(n, (channels + CR_CHANNELS - 1) / CR_CHANNELS), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const uint8_t*>(w), channels, taps,
+                       (channels * taps + CV_BK - 1) / CV_BK * CV_BK, reinterpret_cast<uint16_t*>(out));
     T2H_LAUNCH_CHECK();
     return T2H_OK;
 }

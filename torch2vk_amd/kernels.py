@@ -1177,11 +1177,11 @@ def conv2d_rows(w: torch.Tensor, channels: int, kernel: tuple[int, int]) -> torc
     n, taps = int(w.shape[0]), kernel[0] * kernel[1]
     if w.dtype != torch.uint8 or tuple(w.shape) != (n, -(-channels * taps // 32) * Q8_0_BYTES):
         raise ValueError(f"weight must be uint8 [N, 34 * ceil({channels * taps} / 32)], got {tuple(w.shape)}")
-    blocks = w.reshape(n, -1, Q8_0_BYTES)
-    d = blocks[..., :2].contiguous().view(torch.float16).float()
-    rows = (d * blocks[..., 2:].contiguous().view(torch.int8).float()).view(n, -1)[:, :channels * taps]
-    rows = rows.view(n, channels, taps).transpose(1, 2).reshape(n, -1).to(torch.bfloat16)
-    return torch.nn.functional.pad(rows, (0, -(channels * taps) % 64)).contiguous()
+    w = w.contiguous()
+    _check(w, "weight", torch.uint8, align=2)
+    out = torch.empty(n, -(-channels * taps // 64) * 64, dtype=torch.bfloat16, device=w.device)
+    call("t2h_conv2d_rows_q8_0", ptr(w), n, channels, taps, ptr(out), stream_handle())
+    return out
 
 
 def conv2d(x: torch.Tensor, w_rows: torch.Tensor, bias: torch.Tensor | None, kernel: tuple[int, int], stride: int,

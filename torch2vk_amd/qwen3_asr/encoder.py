@@ -5,9 +5,9 @@ module semantics pytorch_modules.py:452-526), with the MI355X layout:
 
 * conv2d x 3 (3x3, stride 2, pad 1) + bias + GELU as implicit GEMMs (``kernels.conv2d_1ch``, ``kernels.conv2d``):
   activations stay channels-last [chunk, h, w, 480] bf16 and no patch matrix is written.  The second and third
-  convs' weights are laid out tap-major in bf16 once, when the encoder is made (4 MB each).  Other channel counts,
-  and features that are not contiguous fp32, take ``t2h_im2col`` patch rows and one Q8_0 GEMM with the bias and the
-  GELU in its epilogue;
+  convs' weights are laid out tap-major in bf16 before each of them (4 MB), from the packed rows as they are then.
+  Other channel counts, and features that are not contiguous fp32, take ``t2h_im2col`` patch rows and one Q8_0 GEMM
+  with the bias and the GELU in its epilogue;
 * conv_out (no bias) over the (channel, frequency) rows of every time step, with the sinusoidal position
   table added in the GEMM epilogue (fp32 out), then the valid tokens gathered (``index_select``);
 * per layer: LayerNorm -> one Q8_0 GEMM for q|k|v (stacked rows, stacked biases) -> attention within the
@@ -137,12 +137,6 @@ class Qwen3AudioEncoder:
         self.config = weights.config
         if not weights.qkv:
             weights.stack_qkv()
-        c, taps = self.config.conv_channels, CONV_KERNEL * CONV_KERNEL
-        self._conv_rows = {}
-        for name in ("conv2d2", "conv2d3") if c % 8 == 0 and c >= 64 else ():
-            w = weights.packed.get(PREFIX + name + ".weight")
-            if w is not None and tuple(w.shape) == (c, q8_0_cols((c, c * taps)) // 32 * kernels.Q8_0_BYTES):
-                self._conv_rows[name] = kernels.conv2d_rows(w, c, (CONV_KERNEL, CONV_KERNEL))
 
     def _p(self, name: str) -> torch.Tensor:
         return self.weights.packed[PREFIX + name]
@@ -154,18 +148,22 @@ class Qwen3AudioEncoder:
 
     def _conv(self, x: torch.Tensor, name: str) -> torch.Tensor:
         """conv2d (3x3, stride 2, pad 1) + bias + GELU; x channels-last [B, H, W, C] -> bf16 [B, Ho, Wo, Co]."""
-        kernel, bias = (CONV_KERNEL, CONV_KERNEL), self._v(name + ".bias")
+        kernel, weight, bias = (CONV_KERNEL, CONV_KERNEL), self._p(name + ".weight"), self._v(name + ".bias")
         b, h, w, c = x.shape
-        if x.numel() and CONV_KERNEL <= w < 1 << 24 and h < 1 << 24 and w * c < 1 << 28:  # the kernels' 32-bit offsets
-            if name in self._conv_rows:
-                return kernels.conv2d(x, self._conv_rows[name], bias, kernel, CONV_STRIDE, CONV_PAD, act="gelu")
-            if c == 1 and x.dtype == torch.float32 and x.is_contiguous() and self.config.conv_channels % 8 == 0:
-                return kernels.conv2d_1ch(x.view(b, 1, h, w), self._p(name + ".weight"), bias, kernel, CONV_STRIDE,
-                                          CONV_PAD, act="gelu")
+        row_bytes = -(-c * CONV_KERNEL ** 2 // 32) * kernels.Q8_0_BYTES
+        whole = (weight.dtype == torch.uint8 and tuple(weight.shape[1:]) == (row_bytes,) and weight.is_contiguous()
+                 and weight.data_ptr() % 2 == 0 and x.is_contiguous())
+        # (the kernels' 32-bit offsets)
+        if whole and x.numel() and CONV_KERNEL <= w < 1 << 24 and h < 1 << 24 and w * c < 1 << 28:
+            if c >= 64 and c % 8 == 0 and x.dtype == torch.bfloat16:
+                return kernels.conv2d(x, kernels.conv2d_rows(weight, c, kernel), bias, kernel, CONV_STRIDE, CONV_PAD,
+                                      act="gelu")
+            if c == 1 and weight.shape[0] % 8 == 0 and x.dtype == torch.float32:
+                return kernels.conv2d_1ch(x.view(b, 1, h, w), weight, bias, kernel, CONV_STRIDE, CONV_PAD, act="gelu")
         ho = kernels.conv_out_size(h, CONV_KERNEL, CONV_STRIDE, CONV_PAD)
         wo = kernels.conv_out_size(w, CONV_KERNEL, CONV_STRIDE, CONV_PAD)
         cols = kernels.im2col(x.permute(0, 3, 1, 2), kernel, (CONV_STRIDE, CONV_STRIDE), (CONV_PAD, CONV_PAD))
-        y = kernels.q8_0_linear(cols, self._p(name + ".weight"), bias=bias, act="gelu")
+        y = kernels.q8_0_linear(cols, weight, bias=bias, act="gelu")
         return y.view(b, ho, wo, -1)
 
     def frontend(self, padded_feature: torch.Tensor, position_embedding: torch.Tensor) -> torch.Tensor:
