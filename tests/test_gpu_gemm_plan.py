@@ -94,3 +94,86 @@ def test_planned_linear_keeps_unaligned_rows(device):
     odd = buf[2:2 + w.numel()].view(n, -1)
     odd.copy_(w)
     assert torch.equal(kernels.q8_0_linear(x, odd), kernels.q8_0_linear(x, w))
+
+
+def _room_cases(kernels, device):
+    """(name, calls of one planned GEMM each into its own output, one-pass output or None where K is not split)."""
+    g = torch.Generator(device=device)
+    g.manual_seed(6)
+
+    def weights(n, k, wtype):
+        return kernels.quantize(torch.randn(n, k, generator=g, device=device) * 0.05, wtype)
+
+    def x(m, k):
+        return torch.randn(m, k, generator=g, device=device).to(torch.bfloat16)
+
+    m, n, k = 3000, 4100, 2048
+    assert kernels.gemm_plan(m, n, k, "q8_0") == (1, True)
+    x0, w0, y0 = x(m, k), weights(n, k, "q8_0"), torch.empty(m, n, device=device)
+    yield "linear", lambda splits=None: kernels.q8_0_linear(x0, w0, out=y0, out_dtype=torch.float32, splits=splits)
+    yield "gemm", lambda splits=None: kernels.gemm(x0, w0, "q8_0", out=y0, out_dtype=torch.float32, splits=splits)
+    m, n, k = 1900, 6000, 2048
+    assert kernels.gemm_plan(m, n, k, "q4_k", True) == (1, True)
+    x1, w1, w2 = x(m, k), weights(n, k, "q4_k"), weights(n, k, "q4_k")
+    y1 = torch.empty(m, n, dtype=torch.bfloat16, device=device)
+    yield "swiglu", lambda splits=None: kernels.gemm_swiglu(x1, w1, w2, "q4_k", out=y1, splits=splits)
+    m, n, k = 735, 4096, 4096
+    assert kernels.gemm_plan(m, n, k, "q6_k") == (2, True)
+    x3, w3, y3 = x(m, k), weights(n, k, "q6_k"), torch.empty(m, n, device=device)
+    yield "split", lambda splits=None: kernels.gemm(x3, w3, "q6_k", out=y3, out_dtype=torch.float32, splits=splits)
+
+
+@pytest.mark.gpu
+def test_no_room_for_dequantised_rows(device, monkeypatch):
+    """A GEMM whose dequantised rows find no room multiplies the packed rows: the same bits."""
+    from torch2vk_amd import kernels
+
+    def no_room(*args, **kwargs):
+        raise torch.OutOfMemoryError("no room")
+
+    for name, call in _room_cases(kernels, device):
+        want = call().clone()
+        with monkeypatch.context() as m:
+            m.setattr(kernels, "dequantize_bf16", no_room)
+            assert torch.equal(call(), want), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("captured", [False, True])
+def test_no_room_for_any_scratch(device, captured):
+    """With no memory left for a scratch of its size a planned GEMM takes none: one pass over packed rows, eagerly
+    and inside a graph that is replayed."""
+    from torch2vk_amd import kernels
+
+    total = torch.cuda.mem_get_info()[1]
+    cases = list(_room_cases(kernels, device))
+    wants = [call(splits=1).clone() for _, call in cases]  # compiled, and what one pass gives
+    torch.cuda.synchronize()
+    for (name, call), want in zip(cases, wants):
+        planned = call().clone()
+        assert name != "split" or not torch.equal(planned, want)
+        out = call()
+        torch.cuda.empty_cache()
+        filled = []
+        try:
+            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (4 << 20)) / total)
+            with pytest.raises(torch.OutOfMemoryError):
+                while len(filled) < 1000:
+                    filled.append(torch.empty(4 << 20, dtype=torch.uint8, device=device))
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            if captured:
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph):
+                    call()
+            else:
+                call()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.cuda.max_memory_allocated() - before < 4 << 20, name
+        for _ in range(3 if captured else 0):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), name
+        assert torch.equal(out, want), name

@@ -317,14 +317,6 @@ GEMM_FILL_BLOCKS = 128  # from DEQUANT_FIRST_ROWS rows, grids below this many ti
 DEQUANT_FIRST_ROWS = 4096
 
 
-def _dequantized(wtype: str, k: int, *ws: torch.Tensor) -> list[torch.Tensor] | None:
-    """The weights as bf16 scratch, or None when the device has no room for it: the tile loop takes packed rows too."""
-    try:
-        return [dequantize_bf16(w, wtype, k) for w in ws]
-    except torch.OutOfMemoryError:
-        return None
-
-
 def gemm_splits(m: int, n_cols: int, k: int) -> int:
     """K parts for a prefill GEMM of many rows and n_cols tile columns (1 = the one-pass GEMM): when the
     one-pass grid has fewer than GEMM_FILL_BLOCKS tiles, enough parts that the split grid (128-row tiles)
@@ -427,13 +419,36 @@ def _gemm_tiles(wtype: str, x: torch.Tensor, w: torch.Tensor, w_up: torch.Tensor
          ptr(residual), m, k, n, w_k, tile, stream_handle())
 
 
+def _gemm_scratch(m: int, n: int, k: int, wtype: str, splits: int | None, ws: list[torch.Tensor], *,
+                  gated: bool = False, dequant: bool = True) -> tuple[str, list[torch.Tensor], int, torch.Tensor | None]:
+    """What the plan asks for of a GEMM over the weights ``ws``: (type of the rows, rows, K parts, partials).  The rows
+    are bf16 scratch where they are dequantised first, and the partials hold the parts' products.  Where the device has
+    no room for one of them (under capture: the graph's pool) the GEMM runs without, as it did before there were plans:
+    one pass, and packed rows converted in the loop.  Parts that a caller asked for are not given up."""
+    planned = splits is None
+    splits, dequant = _gemm_plan(m, n, k, wtype, splits, gated, dequant)
+    partials = None
+    if splits > 1:
+        nbytes = int(_lib.lib().t2h_gemm_splitk_bytes(m, n, splits, 1 if gated else 0))
+        try:
+            partials = torch.empty(nbytes // 4, dtype=torch.float32, device=ws[0].device)
+        except torch.OutOfMemoryError:
+            if not planned:
+                raise
+            splits = 1
+    if dequant:
+        try:
+            return "bf16", [dequantize_bf16(w, wtype, k) for w in ws], splits, partials
+        except torch.OutOfMemoryError:
+            pass
+    return wtype, ws, splits, partials
+
+
 def _gemm_splitk(wtype: str, x: torch.Tensor, w: torch.Tensor, w_up: torch.Tensor | None, out: torch.Tensor,
-                 m: int, k: int, n: int, w_k: int, splits: int, *, bias: torch.Tensor | None = None, act: int = 0,
-                 residual: torch.Tensor | None = None) -> None:
-    nbytes = int(_lib.lib().t2h_gemm_splitk_bytes(m, n, splits, 1 if w_up is not None else 0))
-    partials = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+                 m: int, k: int, n: int, w_k: int, splits: int, partials: torch.Tensor, *,
+                 bias: torch.Tensor | None = None, act: int = 0, residual: torch.Tensor | None = None) -> None:
     call("t2h_gemm_splitk", WTYPES[wtype], ptr(x), ptr(w), ptr(w_up), ptr(bias), act, ptr(out),
-         _OUT_DTYPES[out.dtype], ptr(residual), m, k, n, w_k, splits, ptr(partials), nbytes, stream_handle())
+         _OUT_DTYPES[out.dtype], ptr(residual), m, k, n, w_k, splits, ptr(partials), partials.numel() * 4, stream_handle())
 
 
 def gemm(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor | None = None,
@@ -464,12 +479,9 @@ def gemm(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor | No
         if tile is not None:
             _gemm_tiles(wtype, x, w, None, out, m, k, n, k, tile, residual=residual)
             return out
-    splits, dequant = _gemm_plan(m, n, k, wtype, splits)
-    dense = _dequantized(wtype, k, w) if dequant else None
-    if dense is not None:
-        (w,), wtype = dense, "bf16"
-    if splits > 1:
-        _gemm_splitk(wtype, x, w, None, out, m, k, n, k, splits, residual=residual)
+    wtype, (w,), splits, partials = _gemm_scratch(m, n, k, wtype, splits, [w])
+    if partials is not None:
+        _gemm_splitk(wtype, x, w, None, out, m, k, n, k, splits, partials, residual=residual)
         return out
     name = {"q8_0": "t2h_q8_0_gemm", "q4_k": "t2h_q4k_gemm", "q6_k": "t2h_q6k_gemm", "bf16": "t2h_bf16_gemm"}[wtype]
     call(name, ptr(x), ptr(w), ptr(out), _OUT_DTYPES[out.dtype], ptr(residual), m, k, n, stream_handle())
@@ -501,12 +513,9 @@ def gemm_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, wtype
         if tile is not None:
             _gemm_tiles(wtype, x, w_gate, w_up, out, m, k, n, k, tile)
             return out
-    splits, dequant = _gemm_plan(m, n, k, wtype, splits, gated=True)
-    dense = _dequantized(wtype, k, w_gate, w_up) if dequant else None
-    if dense is not None:
-        (w_gate, w_up), wtype = dense, "bf16"
-    if splits > 1:
-        _gemm_splitk(wtype, x, w_gate, w_up, out, m, k, n, k, splits)
+    wtype, (w_gate, w_up), splits, partials = _gemm_scratch(m, n, k, wtype, splits, [w_gate, w_up], gated=True)
+    if partials is not None:
+        _gemm_splitk(wtype, x, w_gate, w_up, out, m, k, n, k, splits, partials)
         return out
     call("t2h_gemm_swiglu", WTYPES[wtype], ptr(x), ptr(w_gate), ptr(w_up), ptr(out), m, k, n, stream_handle())
     return out
@@ -657,12 +666,11 @@ def q8_0_linear(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None =
         if tile is not None:
             _gemm_tiles("q8_0", x, w, None, out, m, k, n, w_k, tile, bias=bias, act=ACTS[act], residual=residual)
             return out
-    splits, dequant = _gemm_plan(m, n, k, "q8_0", splits, dequant=w_k == k and w.data_ptr() % 16 == 0)
-    dense, wtype = _dequantized("q8_0", k, w) if dequant else None, "q8_0"
-    if dense is not None:
-        (w,), wtype = dense, "bf16"
-    if splits > 1:
-        _gemm_splitk(wtype, x, w, None, out, m, k, n, w_k, splits, bias=bias, act=ACTS[act], residual=residual)
+    wtype, (w,), splits, partials = _gemm_scratch(m, n, k, "q8_0", splits, [w],
+                                                  dequant=w_k == k and w.data_ptr() % 16 == 0)
+    if partials is not None:
+        _gemm_splitk(wtype, x, w, None, out, m, k, n, w_k, splits, partials, bias=bias, act=ACTS[act],
+                     residual=residual)
     elif wtype == "bf16":
         call("t2h_bf16_linear", ptr(x), ptr(w), ptr(bias), ACTS[act], ptr(out), _OUT_DTYPES[out.dtype], ptr(residual),
              m, k, n, stream_handle())

@@ -477,7 +477,8 @@ class Qwen3Decoder:
         reading the ids from a buffer of the decoder's; later calls copy the ids into that buffer and replay.
         Results are prefill_chunked's bit for bit; a short prompt's prefill is bound by launch overhead, which the
         graph removes.  Each captured graph keeps a memory pool holding every intermediate of one whole prefill
-        (about the GEMM activations of one chunk), so at most PREFILL_GRAPHS of them are kept, least recently
+        (about the GEMM activations of one chunk, and the largest scratch of a GEMM: 2 bytes a value where a layer's
+        weights are dequantised first, 200 MB for the 8B shape's gate|up), so at most PREFILL_GRAPHS of them are kept, least recently
         used first out; ``clear_prefill_graphs`` drops them all."""
         ids = prompt_ids.to(device=self.device, dtype=torch.int64).view(-1)
         if ids.numel() == 0:
