@@ -177,3 +177,23 @@ def test_no_room_for_any_scratch(device, captured):
             torch.cuda.synchronize()
             assert torch.equal(out, want), name
         assert torch.equal(out, want), name
+
+
+def test_plan_below_the_dequantising_rows(monkeypatch):
+    """DEQUANT_FIRST_ROWS is the one limit between the rules, wherever it is set."""
+    from torch2vk_amd import kernels
+
+    n, k = 12288, 4096
+    planned = {m: kernels.gemm_plan(m, n, k, "q4_k") for m in (300, 4095, 6000)}
+    assert kernels._gemm_plan(4095, n, k, "q4_k", None) == planned[4095]
+    assert kernels._gemm_plan(4096, n, k, "q4_k", None) == (1, True)
+    monkeypatch.setattr(kernels, "DEQUANT_FIRST_ROWS", 256)
+    assert kernels._planned(255) and not kernels._planned(256)
+    assert planned[300] != (1, True)
+    assert kernels._gemm_plan(300, n, k, "q4_k", None) == (kernels.gemm_splits(300, n, k), kernels.gemm_splits(300, n, k) == 1)
+    monkeypatch.setattr(kernels, "DEQUANT_FIRST_ROWS", 8192)
+    assert kernels._gemm_plan(6000, n, k, "q4_k", None) == planned[6000]
+    assert kernels._gemm_plan(8192, n, k, "q4_k", None) == (1, True)
+    monkeypatch.setattr(kernels, "DEQUANT_FIRST_ROWS", 0)
+    assert kernels._gemm_plan(300, n, k, "q4_k", None) == (planned[300][0], False)
+    assert kernels._gemm_plan(6000, n, k, "q4_k", None) == (kernels.gemm_splits(6000, n, k), False)

@@ -313,8 +313,14 @@ GEMM_FILL_BLOCKS = 128  # from DEQUANT_FIRST_ROWS rows, grids below this many ti
 # From this many rows of x, a one-pass prefill GEMM always dequantises its packed weights once into a bf16 scratch
 # (t2h_dequantize_bf16) and runs the tile loop on bf16 rows, instead of dequantising every weight tile once per 128 or
 # 256 rows of x inside the loop (measured on MI355X at M 16384, K 4096, N 12288 Q8_0: 1.85 ms in-loop against
-# 0.05 + 1.52 ms); below it gemm_plan decides.  The products are bit-identical either way.  0 disables it.
+# 0.05 + 1.52 ms); below it gemm_tile and gemm_plan decide.  The products are bit-identical either way.  0: no GEMM
+# dequantises first, and those rules hold below their own 4096 rows.
 DEQUANT_FIRST_ROWS = 4096
+
+
+def _planned(m: int) -> bool:
+    """Whether gemm_tile and gemm_plan decide for m rows; more rows split by gemm_splits."""
+    return m < (DEQUANT_FIRST_ROWS or GEMM_TILE_MAX_ROWS + 1)
 
 
 def gemm_splits(m: int, n_cols: int, k: int) -> int:
@@ -330,7 +336,7 @@ def gemm_splits(m: int, n_cols: int, k: int) -> int:
     return max(1, min(k // 128, -(-256 // split_tiles), 16))
 
 
-GEMM_TILE_MAX_ROWS = 4095  # from 4096 rows a dequantised copy of the weights always pays (DEQUANT_FIRST_ROWS)
+GEMM_TILE_MAX_ROWS = 4095  # the rows gemm_tile was measured to, whatever DEQUANT_FIRST_ROWS is
 # Tiles of t2h_gemm_tiles by its ``tile`` argument: rows, columns, the longest K taken.
 GEMM_TILES = ((32, 32, 4096), (64, 32, 4096), (64, 64, 6144), (128, 64, 4096))
 
@@ -405,7 +411,7 @@ def _gemm_plan(m: int, n: int, k: int, wtype: str, splits: int | None, gated: bo
     """(K parts, dequantise first): as the caller gave the parts, by gemm_plan, or from DEQUANT_FIRST_ROWS rows by
     gemm_splits."""
     dequant = dequant and DEQUANT_FIRST_ROWS > 0 and wtype != "bf16"
-    if splits is None and m <= GEMM_TILE_MAX_ROWS:
+    if splits is None and _planned(m):
         return gemm_plan(m, n, k, wtype, gated, dequant)
     if splits is None:
         splits = gemm_splits(m, 2 * n if gated else n, k)
@@ -475,7 +481,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, wtype: str, *, out: torch.Tensor | No
         if residual.numel() != m * n or out.dtype != torch.float32:
             raise ValueError("residual must be fp32 with the output's shape; output must be fp32")
     if splits is None:
-        tile = gemm_tile(m, n, k)
+        tile = gemm_tile(m, n, k) if _planned(m) else None
         if tile is not None:
             _gemm_tiles(wtype, x, w, None, out, m, k, n, k, tile, residual=residual)
             return out
@@ -509,7 +515,7 @@ def gemm_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, wtype
     if out.numel() != m * n:
         raise ValueError(f"output has {out.numel()} elements, expected {m * n}")
     if splits is None:
-        tile = gemm_tile(m, 2 * n, k, True)
+        tile = gemm_tile(m, 2 * n, k, True) if _planned(m) else None
         if tile is not None:
             _gemm_tiles(wtype, x, w_gate, w_up, out, m, k, n, k, tile)
             return out
@@ -662,7 +668,7 @@ def q8_0_linear(x: torch.Tensor, w: torch.Tensor, *, bias: torch.Tensor | None =
         if residual.numel() != m * n or out.dtype != torch.float32:
             raise ValueError("residual must be fp32 with the output's shape; output must be fp32")
     if splits is None:
-        tile = gemm_tile(m, n, k)
+        tile = gemm_tile(m, n, k) if _planned(m) else None
         if tile is not None:
             _gemm_tiles("q8_0", x, w, None, out, m, k, n, w_k, tile, bias=bias, act=ACTS[act], residual=residual)
             return out
