@@ -193,3 +193,21 @@ def test_unmask_schedule():
     sched = unmask_schedule(7, 10)
     assert sum(sched) == 7 and sched[-1] == 0 and all(k >= 0 for k in sched)
     assert unmask_schedule(100, 4)[0] < unmask_schedule(100, 4)[-1]           # shift 0.1: few early, many late
+
+
+def test_codec_chain_keeps_its_offsets_in_32_bits():
+    """t2h_codec_decode takes no decode with an activation of 2^31 or more values, wherever in the chain it is."""
+    import ctypes
+
+    from torch2vk_amd import _lib
+
+    def workspace(dim, latent, hidden, channels, frames):
+        dims = (ctypes.c_uint32 * 7)(1, dim, latent, hidden, channels, 1, 2)
+        return _lib.lib().t2h_codec_decode_workspace_bytes(ctypes.addressof(dims), frames)
+
+    frames = 1 << 21
+    assert workspace(32, 64, 64, 16, frames) > 0
+    assert workspace(32, 1024 - 64, 64, 16, frames) > 0
+    for dim, latent, hidden, channels in ((1024, 64, 64, 16), (32, 1024, 64, 16), (32, 64, 1024, 16), (32, 64, 64, 1024)):
+        assert workspace(dim, latent, hidden, channels, frames) == 0
+        assert workspace(dim, latent, hidden, channels, frames - 1) > 0

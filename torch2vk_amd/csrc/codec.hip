@@ -22,6 +22,8 @@
 #include "codec.h"
 #include "gemm_formats.h"
 
+#include <algorithm>
+
 namespace t2h {
 
 typedef __bf16 cd_bf16x8_t __attribute__((ext_vector_type(8)));
@@ -416,7 +418,9 @@ static int cd_space(const CdDims& d, uint32_t frames, CdSpace& s) {
         const uint64_t n = l * (d.channels >> b);
         s.act = n > s.act ? n : s.act;
     }
-    if (s.act > 0x7fffffffull || (uint64_t)frames * d.books * d.dim > 0x7fffffffull) return T2H_ERR_SHAPE;
+    // every activation of the chain has 32-bit element offsets
+    const uint64_t front = frames * (uint64_t)std::max({d.books * d.dim, d.latent, d.hidden});
+    if (s.act > 0x7fffffffull || front > 0x7fffffffull) return T2H_ERR_SHAPE;
     s.act = up(s.act);
     s.bias = up(4ull * d.latent);
     uint64_t frags = cd_fragments(d.books * d.dim, d.latent, 1) + cd_fragments(d.latent, d.hidden, 1) +
