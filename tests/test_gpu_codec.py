@@ -45,21 +45,11 @@ def test_conv_transpose1d_tiles_match_oracle(device, length, ci, co, k, stride, 
     assert (np.abs(y - ref) <= (n + 2) * 2.0 ** -24 * mag).all()
 
 
-# channels down to 8 (padded column tiles and channel steps), one frame, a frame count past a row tile,
-# channel slabs split over 1, 2 and 4 waves (wide first layers, few rows), more rows than one block takes
-@pytest.mark.parametrize("books,dim,latent,hidden,channels,strides,frames", [
-    (3, 32, 64, 64, 64, (3, 2, 2), 1), (1, 64, 192, 128, 256, (2, 3), 33), (2, 32, 128, 320, 512, (8, 5, 4, 2, 3), 3),
-    (4, 32, 64, 64, 96, (5, 7), 70)])
-def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, channels, strides, frames):
-    """Every stage of the fused decode against the float64 oracle over the stage's own input, and the waveform of
-    the run that keeps no stages against the run that does (the same arithmetic, so the same bits)."""
-    from torch2vk_amd.omnivoice.decoder import AudioDecoderConfig, OmniVoiceAudioDecoder, out_len, synthetic_dense
+def _check_stages(dec, cfg, dense, frames):
+    """Every stage of a decode against the float64 oracle over the stage's own input, and the waveform of the run that
+    keeps no stages against the run that does (the same arithmetic, so the same bits)."""
+    from torch2vk_amd.omnivoice.decoder import out_len
 
-    cfg = AudioDecoderConfig(codebooks=books, vocab=16, codebook_dim=dim, latent=latent, hidden=hidden,
-                             channels=channels, strides=strides)
-    dense = synthetic_dense(cfg, seed=frames)
-    dec = OmniVoiceAudioDecoder(cfg, dense, device)
-    assert dec._plan is not None
     deq = {}
     for n, a in dense.items():
         if a.ndim != 2:
@@ -70,7 +60,7 @@ def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, ch
         if not (n.startswith("cb") or n.endswith("convt.w")):
             deq[n] = R.bf16_round(deq[n].astype(np.float32)).astype(np.float64)
     bf = lambda a: R.bf16_round(np.asarray(a, np.float32)).astype(np.float64)  # noqa: E731
-    codes = np.random.default_rng(8).integers(-1, cfg.vocab + 1, (books, frames)).astype(np.int64)
+    codes = np.random.default_rng(8).integers(-1, cfg.vocab + 1, (cfg.codebooks, frames)).astype(np.int64)
     stages = []
     y = dec.decode(torch.from_numpy(codes), stages=stages)
     assert torch.equal(y, dec.decode(torch.from_numpy(codes)))
@@ -82,7 +72,7 @@ def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, ch
     ids = np.where((codes >= 0) & (codes < cfg.vocab), codes, cfg.vocab)
     checks = [("front", got[0], O.audio_decode_front_ref(cfg, ref_deq, ids, bf))]
     k = 1
-    for i in range(len(strides)):
+    for i in range(len(cfg.strides)):
         checks.append((f"block {i} upsample", got[k], O.audio_decode_upsample_ref(cfg, deq, got[k - 1], i)))
         k += 1
         for j, d in enumerate((1, 3, 9)):
@@ -95,6 +85,34 @@ def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, ch
     for what, a, b in checks:
         assert a.shape == b.shape, what
         assert_close(a, b, max_abs=2.0 ** -8 * float(np.abs(b).max()), min_cos=0.99999, what=what)
+
+
+# channels down to 8 (padded column tiles and channel steps), one frame, a frame count past a row tile,
+# channel slabs split over 1, 2 and 4 waves (wide first layers, few rows), more rows than one block takes
+@pytest.mark.parametrize("books,dim,latent,hidden,channels,strides,frames", [
+    (3, 32, 64, 64, 64, (3, 2, 2), 1), (1, 64, 192, 128, 256, (2, 3), 33), (2, 32, 128, 320, 512, (8, 5, 4, 2, 3), 3),
+    (4, 32, 64, 64, 96, (5, 7), 70)])
+def test_codec_decode_stages_match_oracle(device, books, dim, latent, hidden, channels, strides, frames):
+    """Every stage of the fused decode against the float64 oracle."""
+    from torch2vk_amd.omnivoice.decoder import AudioDecoderConfig, OmniVoiceAudioDecoder, synthetic_dense
+
+    cfg = AudioDecoderConfig(codebooks=books, vocab=16, codebook_dim=dim, latent=latent, hidden=hidden,
+                             channels=channels, strides=strides)
+    dense = synthetic_dense(cfg, seed=frames)
+    dec = OmniVoiceAudioDecoder(cfg, dense, device)
+    assert dec._plan is not None
+    _check_stages(dec, cfg, dense, frames)
+
+
+# latent, hidden and channel sizes that the chain is not built for, more codebooks than it takes, and sizes that it takes
+@pytest.mark.parametrize("fields,fused", [({"latent": 96}, False), ({"hidden": 96}, False), ({"codebooks": 33}, False),
+                                          ({"channels": 48, "strides": (4, 3)}, False), ({"strides": (8, 5)}, True)])
+def test_codec_operators_match_oracle(device, fields, fused):
+    """The decode operator by operator, which runs wherever the chain does not: the same stages, the same oracle."""
+    dec, cfg, dense, _ = _small_codec(device, 41, **fields)
+    assert (dec._plan is not None) == fused
+    dec._plan = None
+    _check_stages(dec, cfg, dense, 11)
 
 
 def _small_codec(device, seed, **fields):
