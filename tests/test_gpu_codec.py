@@ -115,6 +115,19 @@ def test_codec_operators_match_oracle(device, fields, fused):
     _check_stages(dec, cfg, dense, 11)
 
 
+# a 4-column group of an epilogue with one alpha whose argument passes the polynomial's range: the whole group takes
+# the general form, each column its own value
+@pytest.mark.parametrize("column", range(4))
+def test_codec_epilogue_large_arguments(device, column):
+    from torch2vk_amd.omnivoice.decoder import OmniVoiceAudioDecoder
+
+    _, cfg, dense, _ = _small_codec(device, 51)
+    for name in ("b0.alpha", "b0.r0.a2", "b0.r1.a1", "b1.r2.a2", "final.alpha"):
+        dense[name][column::8] = 1e30  # sin^2 / alpha vanishes beside the value
+    dense["b1.r0.a2"][column::8] = 3e9
+    _check_stages(OmniVoiceAudioDecoder(cfg, dense, device), cfg, dense, 13)
+
+
 def _small_codec(device, seed, **fields):
     """A decoder whose shapes the fused chain takes, its dense weights, and codes of one id past its vocab."""
     from torch2vk_amd.omnivoice.decoder import AudioDecoderConfig, OmniVoiceAudioDecoder, synthetic_dense
@@ -190,3 +203,34 @@ def test_codec_decode_reads_the_weights_of_the_call(device, fields):
     a.w["b1.r2.a2"] = a.w["b1.r2.a2"].half()
     with pytest.raises(TypeError):
         a.decode(codes)
+
+
+def test_snake_matches_64_bits(device):
+    """x + sin(alpha x)^2 / (alpha + eps) at the bounds stated for sin^2 (1.2e-7, and 2.8e-7 of its value), alpha a
+    power of two so that its argument is exact.  eps leaves a divisor of 2^-24 alpha, which lifts sin^2 as far above x
+    as 24 bits allow; x's own rounding is what is left at large arguments (2^-18 of sin^2 at 2^30)."""
+    from torch2vk_amd import kernels
+
+    rng = np.random.default_rng(3)
+    near = np.arange(1, 4000) * (np.pi / 2)                    # where the reduced argument is smallest
+    y = np.concatenate([2.0 ** rng.uniform(-20, 30, 20000), near, rng.integers(1, 2 ** 29, 4000) * (np.pi / 2),
+                        [2.0 ** 30, 2.0 ** 30 * (1 + 2.0 ** -23), 1e10, 1e20, 3e38]]).astype(np.float32)
+    y = np.concatenate([y, -y, [0.0]]).astype(np.float32)
+    for alpha in (1.0, 2.0 ** 12, 2.0 ** -6):
+        with np.errstate(over="ignore"):
+            x = (y / np.float32(alpha)).astype(np.float32)
+        ok = np.isfinite(x)
+        x, args = x[ok], y[ok].astype(np.float64)
+        step = 2.0 ** -24 * alpha
+        got = kernels.snake(torch.from_numpy(x).to(device)[:, None].contiguous(),
+                            torch.full((1,), alpha, device=device), eps=-(alpha - step)).cpu().numpy()[:, 0]
+        s2 = np.sin(args) ** 2
+        want = x.astype(np.float64) + s2 / step
+        tol = np.minimum(1.2e-7, 2.8e-7 * s2) / step + 2.0 ** -23 * (np.abs(x.astype(np.float64)) + s2 / step)
+        large = np.abs(args) > 2.0 ** 30
+        tol[large] += 2e-7 / step
+        err = np.abs(got.astype(np.float64) - want)
+        assert (err <= tol).all(), (alpha, args[np.argmax(err - tol)], float((err / tol).max()))
+    bad = torch.tensor([[float("nan")], [float("inf")], [-float("inf")], [1.0]], device=device)
+    out = kernels.snake(bad, torch.ones(1, device=device)).cpu().numpy()[:, 0]
+    assert np.isnan(out[:3]).all() and np.isfinite(out[3])
