@@ -5,7 +5,7 @@
 // A prompt of some hundred tokens or an utterance's encoder frames make grids of 4 to 100 tiles of 128 x 256, so
 // gemm_q_kernel splits K over blocks there, writes fp32 partials and sums them in a second launch.  Here the tiles are small
 // enough to fill the chip in one launch: groups of waves split K inside a block and add their tiles in LDS, and 2
-// or 4 register stages of 128 K are in flight per group.  With so few rows per weight the dequantisation and the
+// or 4 register stages of 128 K are in flight per group, with one stage in LDS (two of any tile exceed its 160 KB).  With so few rows per weight the dequantisation and the
 // LDS traffic of a stage, not the matrix cores, bound a block, and idle CUs the launch.  Measured against the split-K
 // pair (us, weights not in cache): 128 rows, Q4_K: K 1024 N 4096 20.7 -> 7.4; K 2048 N 1024 with residual 15.1 -> 9.3;
 // gate|up K 1024 N 2 x 3072 22.8 -> 9.4; Q6_K K 3072 N 1024 20.5 -> 16.9; 520 rows, Q8_0: K 896 N 2688 26.4 -> 12.9;
@@ -35,9 +35,8 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_tile_kernel(const Gemm
     constexpr int WT = BN * (GT_BK / 32) / GT;  // 32-value weight conversions per thread and stage
     static_assert(AT >= 1 && WT >= 1, "tile too small for its threads");
     constexpr int BUF = (BM + BN) * GT_ROW;
-    constexpr int NBUF = 2 * KS * BUF * 2 <= 160 * 1024 ? 2 : 1;  // LDS: two stages per group where they fit
     constexpr int TS = BN + 8;                  // row of the fp32 result tile
-    constexpr int LDS_BYTES = KS * NBUF * BUF * 2;
+    constexpr int LDS_BYTES = KS * BUF * 2;
     static_assert(KS * BM * TS * 4 <= LDS_BYTES, "the result tiles reuse the stage buffers");
     __shared__ __align__(16) uint8_t lds_raw[LDS_BYTES];
 
@@ -45,12 +44,12 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_tile_kernel(const Gemm
     gt_tile_of(a, tile_m, tile_n);
     const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
     const uint32_t tid = threadIdx.x;
-    const uint32_t kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / GT);  // K group of this wave
+    const uint32_t kg = __builtin_amdgcn_readfirstlane(tid / GT);  // K group of this wave
     const uint32_t t = tid % GT;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave / WN, wn = wave % WN;
-    uint16_t* lds = reinterpret_cast<uint16_t*>(lds_raw) + kg * NBUF * BUF;
+    uint16_t* lds = reinterpret_cast<uint16_t*>(lds_raw) + kg * BUF;
 
     const uint32_t KT = (a.k + GT_BK - 1) / GT_BK;      // stages; group kg takes kg, kg + KS, ...
     const uint32_t NST = (KT + KS - 1) / KS;
@@ -114,35 +113,18 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_tile_kernel(const Gemm
 #pragma unroll
     for (int i = 0; i < RING; ++i)
         load_stage(i, st[i]);
-    if constexpr (NBUF == 2) {
-        store_stage(0, st[0], lds);
-        __syncthreads();
-        for (uint32_t s0 = 0; s0 < NST; s0 += RING) {
+    for (uint32_t s0 = 0; s0 < NST; s0 += RING) {
 #pragma unroll
-            for (int i = 0; i < RING; ++i) {
-                const uint32_t s = s0 + i;
-                if (s >= NST) break;  // block-uniform
-                load_stage(s + RING, st[i]);
-                store_stage(s + 1, st[(i + 1) % RING], lds + ((i + 1) & 1) * BUF);
-                mma_stage(s, lds + (i & 1) * BUF);
-                __syncthreads();
-            }
-        }
-    } else {
-        for (uint32_t s0 = 0; s0 < NST; s0 += RING) {
-#pragma unroll
-            for (int i = 0; i < RING; ++i) {
-                const uint32_t s = s0 + i;
-                if (s >= NST) break;  // block-uniform
-                store_stage(s, st[i], lds);
-                load_stage(s + RING, st[i]);
-                __syncthreads();
-                mma_stage(s, lds);
-                __syncthreads();
-            }
+        for (int i = 0; i < RING; ++i) {
+            const uint32_t s = s0 + i;
+            if (s >= NST) break;  // block-uniform
+            store_stage(s, st[i], lds);
+            load_stage(s + RING, st[i]);
+            __syncthreads();
+            mma_stage(s, lds);
+            __syncthreads();
         }
     }
-    static_assert(RING % 2 == 0, "a stage's LDS buffer is its parity in the ring");
 
     // results through LDS: the K groups' tiles are added there and rows leave in 16-byte pieces
     float* tile = reinterpret_cast<float*>(lds_raw);
