@@ -13,6 +13,7 @@
 //                     the GELU's arithmetic and the output's bytes (128000 pixels, N 480: 58 us for 123 MB, against 92 as
 //                     patch rows and a GEMM).
 #include "gemm_formats.h"
+#include "lds_dma.h"
 
 namespace t2h {
 
@@ -34,24 +35,6 @@ constexpr int CV_ROWB = CV_BK * 2;  // bytes per LDS row of a stage
 
 __device__ __align__(16) const uint8_t conv2d_zeros[16] = {};
 
-// LDS-DMA of 16 B per lane into lds_addr + 16 * lane.  M0 holds the LDS base; one wait state separates its write
-// from the load that reads it.
-__device__ __forceinline__ void cv_dma16(const void* g, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr)
-                 : "memory", "m0");
-}
-// s_waitcnt of the global counter alone (its 6 bits are split over the immediate), and of the LDS counter alone
-template <int N>
-__device__ __forceinline__ void cv_wait_vm() {
-    static_assert(N < 64, "6-bit counter");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | (7 << 4) | (15 << 8));
-}
-__device__ __forceinline__ void cv_wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (3 << 14)); }
-__device__ __forceinline__ void cv_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 // A DMA instruction writes 1 KB of LDS, lane after lane: 8 rows of 128 B.  Of an operand's R rows, instruction g of G =
 // R / 8 brings rows g, g + G, .. and lies 1040 B after the one before: eight lanes read a row's 128 B in order, and a
 // fragment read (one 16-B chunk of 32 consecutive rows) finds 16 consecutive rows in 16 distinct groups of 4 banks.
@@ -73,10 +56,8 @@ __global__ __launch_bounds__(CV_THREADS) void conv2d_kernel(const Conv2dArgs a) 
     constexpr int STEPS = CV_BK / 16;
     __shared__ __align__(16) uint8_t lds[S * STAGE];
 
-    // XCD-contiguous runs of tiles (blocks are dealt to the 8 XCDs round-robin), columns first: the tiles that read
-    // the same pixels share an L2
-    const uint32_t total = a.tiles_m * a.tiles_n, xcd = blockIdx.x % 8, q8 = total / 8, r8 = total % 8;
-    const uint32_t pid = xcd * q8 + min(xcd, r8) + blockIdx.x / 8;
+    // columns first: the tiles that read the same pixels share an L2
+    const uint32_t pid = xcd_run(a.tiles_m * a.tiles_n);
     const uint32_t m0 = pid / a.tiles_n * BM, n0 = pid % a.tiles_n * BN;
 
     const uint32_t t = threadIdx.x;
@@ -133,9 +114,9 @@ __global__ __launch_bounds__(CV_THREADS) void conv2d_kernel(const Conv2dArgs a) 
     auto issue = [&](int q, uint32_t buf) {
         if (q < IA) {
             const uint8_t* g = (inside[q] >> tap) & 1 ? src_a[q] + off : conv2d_zeros;
-            cv_dma16(g, dma_a + buf * STAGE + q * CV_DMA_PITCH);
+            lds_dma16(g, dma_a + buf * STAGE + q * CV_DMA_PITCH);
         } else {
-            cv_dma16(src_w[q - IA] + kb, dma_w + buf * STAGE + (q - IA) * CV_DMA_PITCH);
+            lds_dma16(src_w[q - IA] + kb, dma_w + buf * STAGE + (q - IA) * CV_DMA_PITCH);
         }
         if (q == DMA - 1) advance();
     };
@@ -184,8 +165,8 @@ __global__ __launch_bounds__(CV_THREADS) void conv2d_kernel(const Conv2dArgs a) 
 #pragma unroll
         for (int q = 0; q < DMA; ++q) issue(q, s);
     }
-    cv_wait_vm<(S - 1) * DMA>();
-    cv_barrier();
+    wait_vm<(S - 1) * DMA>();
+    wave_barrier();
     read_step(0, 0, 0);
     uint32_t buf = 0;
     for (uint32_t kt = 0; kt + 1 < KT; ++kt) {
@@ -195,9 +176,9 @@ __global__ __launch_bounds__(CV_THREADS) void conv2d_kernel(const Conv2dArgs a) 
             mma_step(step & 1);
         }
         // stage kt + 1 landed (every wave's DMA), stage kt's reads done (every wave)
-        cv_wait_vm<(S - 2) * DMA>();
-        cv_wait_lgkm0();
-        cv_barrier();
+        wait_vm<(S - 2) * DMA>();
+        wait_lgkm0();
+        wave_barrier();
         const uint32_t next = buf + 1 == S ? 0 : buf + 1;
         read_step(next, 0, 0);
         constexpr int MM = MI * NJ;
@@ -215,7 +196,7 @@ __global__ __launch_bounds__(CV_THREADS) void conv2d_kernel(const Conv2dArgs a) 
         if (step + 1 < STEPS) read_step(buf, step + 1, (step + 1) & 1);
         mma_step(step & 1);
     }
-    cv_wait_vm<0>();  // the stages issued past the end still write LDS
+    wait_vm<0>();  // the stages issued past the end still write LDS
 
     // lane holds column (lane % 32) of each 32 x 32 tile, rows 8(e/4) + 4(lane/32) + e%4
     const uint32_t row_base = m0 + wm * 32 * MI + (lane >> 5) * 4;

@@ -28,6 +28,13 @@ struct GemmArgs {
     uint32_t vec;          // gemm_tile_kernel: rows of C and the residual can be accessed 4 values at a time
 };
 
+// The tile of `total` that this block computes: blocks are dealt round-robin to the 8 XCDs, and each XCD takes a
+// contiguous run of tiles.
+__device__ __forceinline__ uint32_t xcd_run(uint32_t total) {
+    const uint32_t xcd = blockIdx.x % 8;
+    return xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+}
+
 // Packed row of B-tile row r (0..255) of the tile at n0.  Plain: weight row
 // n0 + r.  Gated (SwiGLU): each wave's 64 columns are 32 gate rows then the 32
 // up rows of the same features, so the epilogue finds g and u in one lane:

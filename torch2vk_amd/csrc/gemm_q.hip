@@ -27,6 +27,7 @@
 // remapped so that each XCD walks a contiguous run of tiles, grouped 8 tiles
 // down M, so the A rows and weight rows a group shares stay in that XCD's L2.
 #include "gemm_formats.h"
+#include "lds_dma.h"
 
 #include <type_traits>
 
@@ -342,14 +343,6 @@ constexpr int GR_ROWB = GQ_BK * 2;            // bytes per LDS row of a stage
 constexpr int GR_STAGE = 2 * 256 * GR_ROWB;   // A rows then W rows: 64 KB
 constexpr int GR_IPW = 256 * GR_ROWB / 1024 / 4;  // 1-KB DMA instructions per wave per operand and stage
 
-// LDS-DMA of 16 B per lane into lds_addr + 16 * lane.  M0 holds the LDS base; one wait state separates its
-// write from the load that reads it.
-__device__ __forceinline__ void gr_dma16(const void* g, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_addr)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void gr_wait_vm0() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
-__device__ __forceinline__ void gr_wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (3 << 14)); }
 // slot of 16-B chunk c in LDS row r is c ^ gr_swizzle(r)
 __device__ __forceinline__ uint32_t gr_swizzle(uint32_t r) { return (r & 7) ^ ((r >> 3) & 1); }
 
@@ -406,10 +399,10 @@ __global__ __launch_bounds__(GR_THREADS) void gemm_bf16_ring_kernel(const GemmAr
     auto issue_stage = [&](uint32_t kt, uint32_t buf) {
         const uint32_t kb = kt * GR_ROWB;
 #pragma unroll
-        for (int i = 0; i < GR_IPW; ++i) gr_dma16(src_a[i] + kb, dma_base + buf * GR_STAGE + i * 1024);
+        for (int i = 0; i < GR_IPW; ++i) lds_dma16(src_a[i] + kb, dma_base + buf * GR_STAGE + i * 1024);
 #pragma unroll
         for (int i = 0; i < GR_IPW; ++i)
-            gr_dma16(src_w[i] + kb, dma_base + buf * GR_STAGE + 256 * GR_ROWB + i * 1024);
+            lds_dma16(src_w[i] + kb, dma_base + buf * GR_STAGE + 256 * GR_ROWB + i * 1024);
     };
     // one 16-deep step: the next step's 8 fragment reads interleaved with the 16 MFMAs
     auto mma_step = [&](int b) {
@@ -435,9 +428,9 @@ __global__ __launch_bounds__(GR_THREADS) void gemm_bf16_ring_kernel(const GemmAr
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[b][i], fb[b][j], acc[i][j], 0, 0, 0);
                 const int q = i * 4 + j;
                 if (q < GR_IPW)
-                    gr_dma16(src_a[q] + kb, dma_base + buf * GR_STAGE + q * 1024);
+                    lds_dma16(src_a[q] + kb, dma_base + buf * GR_STAGE + q * 1024);
                 else
-                    gr_dma16(src_w[q - GR_IPW] + kb, dma_base + buf * GR_STAGE + 256 * GR_ROWB + (q - GR_IPW) * 1024);
+                    lds_dma16(src_w[q - GR_IPW] + kb, dma_base + buf * GR_STAGE + 256 * GR_ROWB + (q - GR_IPW) * 1024);
             }
     };
     static_assert(2 * GR_IPW == 16, "one DMA instruction per MFMA of a step");
@@ -445,10 +438,8 @@ __global__ __launch_bounds__(GR_THREADS) void gemm_bf16_ring_kernel(const GemmAr
     // Stage kt lives in buffer kt % 2.  Every iteration issues one stage's DMA, clamped to the last stage past
     // the end (into a buffer nothing reads again), so the wait before each barrier is the same.
     issue_stage(0, 0);
-    gr_wait_vm0();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    wait_vm<0>();
+    wave_barrier();
     issue_stage(min(1u, KT - 1), 1);
     read_step(0, 0, 0);
     constexpr int STEPS = GQ_BK / 16;
@@ -460,11 +451,9 @@ __global__ __launch_bounds__(GR_THREADS) void gemm_bf16_ring_kernel(const GemmAr
             mma_step(step & 1);
         }
         // stage kt + 1 landed (every wave's DMA), stage kt's reads done (every wave): buffer buf is free
-        gr_wait_vm0();
-        gr_wait_lgkm0();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        wait_vm<0>();
+        wait_lgkm0();
+        wave_barrier();
         read_step(buf ^ 1, 0, 0);
         mma_step_dma((STEPS - 1) & 1, min(kt + 2, KT - 1), buf);
     }
@@ -477,7 +466,7 @@ __global__ __launch_bounds__(GR_THREADS) void gemm_bf16_ring_kernel(const GemmAr
         }
         mma_step((STEPS - 1) & 1);
     }
-    gr_wait_vm0();  // the clamped DMA of the last iteration lands before the block's LDS is released
+    wait_vm<0>();  // the clamped DMA of the last iteration lands before the block's LDS is released
 
     // epilogue: lane holds column (lane % 32) of each 32 x 32 tile, rows 8 (e / 4) + 4 (lane / 32) + e % 4
     const uint32_t row_base = m0 + wm * 128 + (lane >> 5) * 4;

@@ -17,11 +17,9 @@ namespace t2h {
 constexpr int GT_BK = 128;
 constexpr int GT_ROW = GT_BK + 8;  // LDS row: 16-byte reads of 16 consecutive rows hit 16 distinct 4-bank groups
 
-// The block's tile: blocks are dealt round-robin to the 8 XCDs; each XCD takes a contiguous run of tiles, M fastest,
-// so the M tiles that share weight rows share an L2.
+// The block's tile, M fastest, so the M tiles that share weight rows share an L2.
 __device__ __forceinline__ void gt_tile_of(const GemmArgs& a, uint32_t& tile_m, uint32_t& tile_n) {
-    const uint32_t total = a.tiles_m * a.tiles_n, x = blockIdx.x % 8, j = blockIdx.x / 8;
-    const uint32_t i = x * (total / 8) + min(x, total % 8) + j;
+    const uint32_t i = xcd_run(a.tiles_m * a.tiles_n);
     tile_m = i % a.tiles_m;
     tile_n = i / a.tiles_m;
 }
