@@ -197,3 +197,14 @@ def test_plan_below_the_dequantising_rows(monkeypatch):
     monkeypatch.setattr(kernels, "DEQUANT_FIRST_ROWS", 0)
     assert kernels._gemm_plan(300, n, k, "q4_k", None) == (planned[300][0], False)
     assert kernels._gemm_plan(6000, n, k, "q4_k", None) == (kernels.gemm_splits(6000, n, k), False)
+
+
+def test_tiles_leave_long_chains_to_split_k():
+    """Few blocks of 64 x 64 or 128 x 64 over a long K are slower than splits over the idle CUs (up to 1.5 times)."""
+    from torch2vk_amd import kernels
+
+    for m, n_cols, k in ((118, 2 * 2688, 6144), (350, 2 * 1024, 5120), (69, 2 * 4035, 4096), (92, 2 * 4608, 3328),
+                         (27, 2 * 2048, 1792), (42, 2 * 2048, 2048)):
+        assert kernels.gemm_tile(m, n_cols, k, True) is None, (m, n_cols, k)
+    assert kernels.gemm_tile(128, 2 * 3072, 1024, True) == 2 and kernels.gemm_tile(115, 2 * 6144, 2048, True) == 3
+    assert kernels.gemm_tile(64, 2048, 4096) == 0 and kernels.gemm_tile(520, 896, 3584) == 1

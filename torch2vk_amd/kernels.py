@@ -338,7 +338,9 @@ def gemm_splits(m: int, n_cols: int, k: int) -> int:
 
 GEMM_TILE_MAX_ROWS = 4095  # the rows gemm_tile was measured to, whatever DEQUANT_FIRST_ROWS is
 # Tiles of t2h_gemm_tiles by its ``tile`` argument: rows, columns, the longest K taken.
-GEMM_TILES = ((32, 32, 4096), (64, 32, 4096), (64, 64, 6144), (128, 64, 4096))
+GEMM_TILES = ((32, 32, 4096), (64, 32, 4096), (64, 64, 3840), (128, 64, 2816))
+# and the longest K below so many blocks: the fewer the CUs at work, the sooner split-K over the idle ones is faster
+_GEMM_TILE_SHORT = {2: ((72, 1536), (128, 2048), (192, 2816)), 3: ((192, 2304),)}
 
 
 @functools.lru_cache(maxsize=4096)
@@ -346,12 +348,14 @@ def gemm_tile(m: int, n_cols: int, k: int, gated: bool = False) -> int | None:
     """The t2h_gemm_tiles tile for a prefill GEMM of m rows and n_cols tile columns, or None (the 128- and 256-row
     tiles of gemm_q_kernel): the smallest tile whose grid is one block per CU (a block fills a CU's LDS, so a
     second round costs as much as the first), else up to K 1024 128 x 64 in up to two rounds.  A longer K than the tile's
-    is a serial chain that split-K over idle CUs beats.  Measured (us, tile against split-K or one pass): 128 rows K 1024
-    N 4096, 256 blocks of 64 x 32: 7.4 against 20.7, of 64 x 64 (128 blocks): 9.3; 300 rows: 128 x 64 (192 blocks) 13.6,
-    64 x 64 (320) 17.3, split-K 30.6; 520 rows, K 1024 N 2 x 3072: 128 x 64 (480 blocks) 23.6 against 36.3; 1024 rows, the same
-    (768 blocks): 35.3 against 27.5; 548 rows K 4096 N 4096, 320 blocks: 66 against 49 in 3 splits; 128 rows K 6144 N 2048: 64 x 32 25.2 against
-    22.7; Q6_K K 12288 N 4096: 62 against 47; 22 rows gate|up K 6144 N 2 x 2048, 64 blocks of 64 x 64: 40 against 23.  Over 145 random
-    shapes of 9 to 4000 rows the tiles take 0.74 of the time."""
+    is a serial chain that split-K over idle CUs beats: a stage of 128 K a group of waves is about 2.3 us, with 8, 4, 4 and
+    2 groups.  Measured (us, tile against split-K or one pass): 128 rows K 1024 N 4096, 256 blocks of 64 x 32: 7.4 against
+    20.7, of 64 x 64 (128 blocks): 9.3; 300 rows: 128 x 64 (192 blocks) 13.6, 64 x 64 (320) 17.3, split-K 30.6; 520 rows,
+    K 1024 N 2 x 3072: 128 x 64 (480 blocks) 23.6 against 36.3; 1024 rows, the same (768 blocks): 35.3 against 27.5; 548 rows
+    K 4096 N 4096, 320 blocks: 66 against 49 in 3 splits.  Past the limits: 64 x 64 in 168 blocks, K 6144: 40 against 27;
+    in 64, K 1792: 14.4 against 12.9; 128 x 64 in 172, K 3328: 34.4 against 28.2; in 144, K 3584: 33.3 against 27.2.
+    Over 2033 random shapes of 9 to 700 rows, K 1024 to 6656, the choice takes 1.011 of the faster of the two and 0.79 of
+    the time that splits by gemm_splits take, at worst 1.13 of it."""
     if m > GEMM_TILE_MAX_ROWS:
         return None
     blocks = 0
@@ -360,7 +364,8 @@ def gemm_tile(m: int, n_cols: int, k: int, gated: bool = False) -> int | None:
             continue
         blocks = -(-m // rows) * -(-n_cols // cols)
         if blocks <= 256:
-            return tile if k <= (2048 if tile == 2 and blocks < 160 else k_max) else None
+            return tile if k <= next((limit for below, limit in _GEMM_TILE_SHORT.get(tile, ()) if blocks < below), k_max) \
+                else None
     if k <= 1024 and blocks <= 512:
         return len(GEMM_TILES) - 1
     return None
