@@ -335,7 +335,11 @@ static void cd_launch(const CdConvArgs& a, hipStream_t s) {
 }
 
 // The fewest waves per row tile (the most rows per weight fragment) that still gives about a block per CU, at
-// most one per slab of channels; one column tile per block only where there is one, or too few blocks of two.
+// most one per slab of channels; one column tile per block only where there is one, or too few blocks of two.  Measured
+// over the codec's 34 convolutions (us, this rule / the fastest of the six forms for each layer): 1 frame 160 / 143,
+// 12: 171 / 152, 75: 281 / 251, 200: 447 / 423, 500: 901 / 855, 1500: 2534 / 2496.  What it leaves are narrow layers of
+// few blocks, where one column tile a block and a split past one wave per slab are faster (600 rows of 512, 7 taps: 10.5
+// in 152 blocks of two tiles, 9.5 in 304 of one; 12000 of 128: 11.7 against 9.6; 960 of 32: 5.5 against 4.2 over 4 waves).
 template <int TAPS, int SC>
 static void cd_dispatch(const CdConvArgs& a, hipStream_t s) {
     const uint32_t slabs = (a.ksteps * 16 + SC - 1) / SC;

@@ -4,14 +4,16 @@
 //   conv2d_kernel     C >= 64 input channels.  Weight rows are bf16 and tap-major (k = tap * C + channel, zero-padded to
 //                     a whole 64-deep stage), so a 16-B chunk of a stage is 8 channels of one tap: the LDS-DMA that
 //                     brings a stage reads it straight from the activation, or from zeros where the tap is outside.
-//                     Bound by the matrix cores and, at 256 x 256 tiles, by one wave a SIMD issuing both the DMA and
-//                     the products: 32000 pixels of C 480, N 480 in 142 us (930 TFLOP/s) against 421 us as a patch
-//                     matrix (276 MB) and a GEMM, 8320 pixels in 62 against 132, 208 pixels in 21 against 28.  Tried:
-//                     32-deep stages that walk the 9 taps of 32 channels at a time (fewer bytes from HBM, but 64-B
-//                     requests run at two thirds of the L2's rate): 141 at 32000 pixels, 67 at 8320, 30 at 208.
+//                     At 256 x 256 tiles one wave a SIMD issues both the DMA and the products, and the matrix cores
+//                     are busy 43 % of the launch (250 tiles, waits 15 % of the waves' cycles); at 128 x 128 22 %,
+//                     LDS 22 % (half of it bank conflicts), waits 43 %.  32000 pixels of C 480, N 480 in 142 us
+//                     (930 TFLOP/s) against 421 us as a patch matrix (276 MB) and a GEMM, 8320 pixels in 62 against
+//                     132, 208 pixels in 21 against 28.  Tried: 32-deep stages that walk the 9 taps of 32 channels at a
+//                     time (fewer bytes from HBM, but 64-B requests run at two thirds of the L2's rate): 141 at 32000
+//                     pixels, 67 at 8320, 30 at 208.
 //   conv2d_1ch_kernel one fp32 input channel (the mel spectrogram): the at most 16 taps are one MFMA step; bound by
-//                     the GELU's arithmetic and the output's bytes (128000 pixels, N 480: 58 us for 123 MB, against 92 as
-//                     patch rows and a GEMM).
+//                     the GELU's arithmetic (VALU busy three quarters of the launch) and the output's bytes (128000
+//                     pixels, N 480: 58 us for 123 MB, against 92 as patch rows and a GEMM).
 #include "gemm_formats.h"
 #include "lds_dma.h"
 
@@ -37,7 +39,8 @@ __device__ __align__(16) const uint8_t conv2d_zeros[16] = {};
 
 // A DMA instruction writes 1 KB of LDS, lane after lane: 8 rows of 128 B.  Of an operand's R rows, instruction g of G =
 // R / 8 brings rows g, g + G, .. and lies 1040 B after the one before: eight lanes read a row's 128 B in order, and a
-// fragment read (one 16-B chunk of 32 consecutive rows) finds 16 consecutive rows in 16 distinct groups of 4 banks.
+// fragment read (one 16-B chunk of 32 consecutive rows) finds 16 consecutive rows in 16 distinct groups of 4 banks.  At
+// 256 rows no conflicts are counted; at 128, where rows 16 to 31 lie 128 B after rows 0 to 15, half of the LDS cycles.
 constexpr int CV_DMA_PITCH = 1024 + 16;
 __device__ __forceinline__ constexpr uint32_t cv_lds_row(uint32_t r, uint32_t G) {
     return r % G * CV_DMA_PITCH + r / G * CV_ROWB;
@@ -415,6 +418,9 @@ extern "C" int t2h_conv2d_bf16(const void* x, const void* w_rows, const void* bi
     //   208 rows 21 / 39 / 39 / 106      3120 rows 29 / 40 / 49 / 110     4160 rows 40 / 42 / 50 / 110
     //   6240 rows 56 / 41 / 49 / 110     8000 rows 66 / 49 / 60 / 122    12000 rows 92 / 86 / 75 / 123
     //   24000 rows 178 / 134 / 131 / 128 32000 rows 237 / 177 / 156 / 142
+    // C = N 64, 128, 256 and 768 at 56 to 48000 rows: within 6 % of the fastest of the four, but for two of the 40:
+    // 8320 rows of 256 (26.7 against 22.9 as 64 x 64) and 48000 of 64, half of whose 128 columns are padding (18.8
+    // against 11.9)
     if (tile < 0) {
         const uint64_t t64 = ((m + 63) / 64) * ((n + 63) / 64), t128 = ((m + 127) / 128) * ((n + 127) / 128);
         const uint64_t t256 = ((m + 255) / 256) * ((n + 255) / 256);

@@ -37,11 +37,12 @@ struct ConvTArgs {
 // One block: 32 rows i (the first `halo` of them only feed the others' outputs) x nt column tiles of 32
 // entries e, one wave per column tile, so a tile's B operand is exactly one Q8_0 block per channel and nt K is
 // a whole number of output channels: the fold needs nothing from other blocks and G never leaves LDS.
-// Channels stream through LDS 32 at a time, CT_RING - 1 stages of loads in flight to registers.  The bound is the
-// CU: a wave and stage is 16 MFMAs of 64 cycles, and staging B (dequantising 16 values a lane, writing and
-// reading them once in LDS) costs about as much again for a tile of only 32 rows.  Measured over the codec's five
-// upsampling layers at 75 frames (1024 to 64 channels, strides 8, 5, 4, 2, 3; 5.8 GFLOP): 2917 us for the
-// per-output kernel below, 157 us here (36 + 41 + 32 + 21 + 25).
+// Channels stream through LDS 32 at a time, CT_RING - 1 stages of loads in flight to registers.  What bounds a block is
+// its chain of stages: a wave and stage is 16 MFMAs of 64 cycles, and staging B (dequantising 16 values a lane, writing
+// and reading them once in LDS) comes before them for a tile of only 32 rows.  Measured over the codec's five upsampling
+// layers at 75 frames (1024 to 64 channels, strides 8, 5, 4, 2, 3; 5.8 GFLOP): 2917 us for the per-output kernel below,
+// 160 us here (36 + 41 + 33 + 24 + 26).  Counters of the first, second, third and last: matrix cores busy 24, 23, 18 and
+// 11 % of the launch, LDS 17, 14, 16 and 9 %, waves waiting 28, 37, 29 and 43 % of their cycles; the first fills 192 CUs.
 constexpr int CT_ROWS = 32;     // rows of G per block
 constexpr int CT_CB = 32;       // channels per LDS stage
 constexpr int CT_MAX_NT = 8;

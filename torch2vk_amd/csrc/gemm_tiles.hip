@@ -5,11 +5,12 @@
 // A prompt of some hundred tokens or an utterance's encoder frames make grids of 4 to 100 tiles of 128 x 256, so
 // gemm_q_kernel splits K over blocks there, writes fp32 partials and sums them in a second launch.  Here the tiles are small
 // enough to fill the chip in one launch: groups of waves split K inside a block and add their tiles in LDS, and 2
-// or 4 register stages of 128 K are in flight per group, with one stage in LDS (two of any tile exceed its 160 KB).  With so few rows per weight the dequantisation and the
-// LDS traffic of a stage, not the matrix cores, bound a block, and idle CUs the launch.  Measured against the split-K
-// pair (us, weights not in cache): 128 rows, Q4_K: K 1024 N 4096 20.7 -> 7.4; K 2048 N 1024 with residual 15.1 -> 9.3;
-// gate|up K 1024 N 2 x 3072 22.8 -> 9.4; Q6_K K 3072 N 1024 20.5 -> 16.9; 520 rows, Q8_0: K 896 N 2688 26.4 -> 12.9;
-// K 3584 N 896 21.8 -> 17.3.
+// or 4 register stages of 128 K are in flight per group, with one stage in LDS (two of any tile exceed its 160 KB).
+// What bounds a block is the chain of its stages (loads, conversion, LDS, barrier, products) at two waves a SIMD, and
+// idle CUs the launch: counters over the shapes below show the matrix cores busy 1 to 6 %, LDS 3 to 19 % and waves
+// waiting 29 to 47 % of their cycles.  Measured against the split-K pair (us, weights not in cache): 128 rows, Q4_K:
+// K 1024 N 4096 20.7 -> 7.4; K 2048 N 1024 with residual 15.1 -> 9.3; gate|up K 1024 N 2 x 3072 22.8 -> 9.4; Q6_K K 3072
+// N 1024 20.5 -> 16.9; 520 rows, Q8_0: K 896 N 2688 26.4 -> 12.9; K 3584 N 896 21.8 -> 17.3.
 #include "gemm_formats.h"
 
 namespace t2h {

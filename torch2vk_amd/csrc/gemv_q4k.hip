@@ -578,7 +578,8 @@ extern "C" int t2h_q4k_matvec(const void* x, const void* w, void* y, int out_dty
     // Every token in one launch, blockIdx.y its row: the tokens' blocks run side by side, so the weights come from
     // HBM once and from L2 for the others (block x of every token runs on the same XCD where the grid is a multiple
     // of 8 blocks), and one token's latencies hide the next's.  6 tokens of K 4096, N 4096: 9.9 us (20.3 as 6
-    // launches), of K 1024, N 3072: 4.5 (16.1).
+    // launches), of K 1024, N 3072: 4.5 (16.1); with other weights each call, past the 256 MB cache, 10.3 (21.4) and 4.6
+    // (16.3).
     for (uint32_t row = 0; row < m; row += 65535) {
         Q4GemvArgs a = {};
         const void* wv[1] = {w};
