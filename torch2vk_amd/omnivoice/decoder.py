@@ -18,7 +18,8 @@ from __future__ import annotations
 import ctypes
 import math
 from dataclasses import dataclass
-from operator import attrgetter, itemgetter
+from functools import reduce
+from operator import attrgetter, itemgetter, or_
 
 import numpy as np
 import torch
@@ -116,7 +117,7 @@ class _Operands:
         self.dtypes = [torch.float32 if len(s) == 1 else torch.uint8 for _, s in shapes]
         self.sizes = [s if len(s) == 1 else (s[0], -(-s[1] // 32) * kernels.Q8_0_BYTES) for _, s in shapes]
         self.tables = [i for i, (name, _) in enumerate(shapes) if name.startswith("cb")]  # of any number of rows
-        self.vectors = [i for i, (_, s) in enumerate(shapes) if len(s) == 1]
+        self.vectors = itemgetter(*(i for i, (_, s) in enumerate(shapes) if len(s) == 1))
 
     def pointers(self, w: dict[str, torch.Tensor]) -> tuple[list[int], list[int]] | None:
         """(pointers, rows of the codebooks), or None where a weight is not as the chain reads it.  Looked at on every
@@ -137,7 +138,7 @@ class _Operands:
         if sizes != self.sizes or not all(map(_is_cuda, ts)) or not all(map(torch.Tensor.is_contiguous, ts)):
             return None
         ptrs = list(map(torch.Tensor.data_ptr, ts))
-        if any(p & 1 for p in ptrs) or any(ptrs[i] & 15 for i in self.vectors) or 0 in ptrs:
+        if reduce(or_, ptrs) & 1 or reduce(or_, self.vectors(ptrs)) & 15 or 0 in ptrs:
             return None
         return ptrs, rows
 
