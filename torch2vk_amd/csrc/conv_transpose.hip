@@ -41,8 +41,8 @@ struct ConvTArgs {
 // its chain of stages: a wave and stage is 16 MFMAs of 64 cycles, and staging B (dequantising 16 values a lane, writing
 // and reading them once in LDS) comes before them for a tile of only 32 rows.  Measured over the codec's five upsampling
 // layers at 75 frames (1024 to 64 channels, strides 8, 5, 4, 2, 3; 5.8 GFLOP): 2917 us for the per-output kernel below,
-// 160 us here (36 + 41 + 33 + 24 + 26).  Counters of the first, second, third and last: matrix cores busy 24, 23, 18 and
-// 11 % of the launch, LDS 17, 14, 16 and 9 %, waves waiting 28, 37, 29 and 43 % of their cycles; the first fills 192 CUs.
+// 160 us here (36 + 41 + 33 + 24 + 26).  Counters of the first, second, fourth and last: matrix cores busy 24, 23, 18
+// and 11 % of the launch, LDS 17, 14, 16 and 9 %, waves waiting 28, 37, 29 and 43 % of their cycles; the first fills 192 CUs.
 constexpr int CT_ROWS = 32;     // rows of G per block
 constexpr int CT_CB = 32;       // channels per LDS stage
 constexpr int CT_MAX_NT = 8;
